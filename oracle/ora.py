@@ -34,7 +34,7 @@ def build(with_ref=None):
     """Compile the oracle (and oracle/_ref when the reference tree exists)."""
     subprocess.run(["make", "-s", "-C", HERE, "all"], check=True)
     if with_ref is None:
-        with_ref = os.path.isdir(REFERENCE_TREE)
+        with_ref = os.path.exists(os.path.join(REFERENCE_TREE, "sampling", "halton.cpp"))
     if with_ref:
         subprocess.run(["make", "-s", "-C", HERE, "ref", f"REF={REFERENCE_TREE}"], check=True)
 
