@@ -169,11 +169,11 @@ PSY_DEV bool patch_box_ray(V3 lo, V3 hi, V3 o, V3 dinv, float t, float* h0, floa
 }
 
 // How a trace handles a patch node that needs splits below the dice cache:
-// D_FLAG flags the ray for the second pass (main pass), D_SERIAL splits on
-// in the lane within a node budget (second pass; a ray that runs out of
-// budget is flagged for the third pass), D_COOP splits with the 64 lanes of
-// the wave together (third pass: every lane runs the same ray).
-constexpr int D_FLAG = 0, D_SERIAL = 1, D_COOP = 2;
+// D_SERIAL splits on in the lane within a node budget (second pass; a ray
+// that runs out of budget is flagged for the third pass), D_COOP splits with
+// the 64 lanes of the wave together (third pass: every lane runs the same
+// ray).  (The main pass's own walk, lane_step, lists such nodes instead.)
+constexpr int D_SERIAL = 1, D_COOP = 2;
 struct DeepState {
     bool need;          // flagged for the next pass
     int32_t budget;     // D_SERIAL: node expansions left
@@ -450,12 +450,9 @@ __device__ bool dice_deep_coop(const DevScene& s, const DevObject& ob, uint32_t 
 }
 
 template <int DEEP>
-PSY_DEV bool deep_or_flag(const DevScene& s, const DevObject& ob, uint32_t k, uint32_t inst, V3 o,
+PSY_DEV bool deep_walk(const DevScene& s, const DevObject& ob, uint32_t k, uint32_t inst, V3 o,
                                              V3 dinv, const RayW& w, bool occl, Best& b, DeepState& ds) {
-    if constexpr (DEEP == D_FLAG) {
-        ds.need = true;
-        return false;
-    } else if constexpr (DEEP == D_COOP) {
+    if constexpr (DEEP == D_COOP) {
         return ob.kind == K_BILINEAR ? dice_deep_coop<4>(s, ob, k, inst, o, dinv, w, occl, b, ds.coop)
                                      : dice_deep_coop<16>(s, ob, k, inst, o, dinv, w, occl, b, ds.coop);
     } else {
@@ -482,7 +479,7 @@ PSY_DEV bool dice_walk(const DevScene& s, const DevObject& ob, uint32_t inst, V3
         const float maxd = longest_axis(sub(xyz(c), xyz(a)));
         if (maxd <= dice_width(min_width(w, h0, h1) * s.dice_rate, s.min_upoly))
             return accept_leaf(h0, h1, a.w, c.w, maxd, inst, b) && occl;
-        if (levels == 0) return deep_or_flag<DEEP>(s, ob, 1, inst, o, dinv, w, occl, b, need_deep);
+        if (levels == 0) return deep_walk<DEEP>(s, ob, 1, inst, o, dinv, w, occl, b, need_deep);
     }
     uint32_t k = 1;
     int depth = 0;
@@ -516,8 +513,8 @@ PSY_DEV bool dice_walk(const DevScene& s, const DevObject& ob, uint32_t inst, V3
         split1 = split1 && h10 <= b.t;
         const int cd = depth + 1;
         if (cd == levels) {
-            if (split1 && deep_or_flag<DEEP>(s, ob, c0 + 1, inst, o, dinv, w, occl, b, need_deep)) return true;
-            if (split0 && deep_or_flag<DEEP>(s, ob, c0, inst, o, dinv, w, occl, b, need_deep)) return true;
+            if (split1 && deep_walk<DEEP>(s, ob, c0 + 1, inst, o, dinv, w, occl, b, need_deep)) return true;
+            if (split0 && deep_walk<DEEP>(s, ob, c0, inst, o, dinv, w, occl, b, need_deep)) return true;
             split0 = split1 = false;
         }
         if (split0 && split1) {
@@ -656,53 +653,60 @@ PSY_DEV void node_boxes(const DevScene& s, int32_t ref, float time, bool ds0, bo
     }
 }
 
+// A sphere, sphere light or rectangle light in the leaf's space; true when
+// an occlusion ray is done.
+PSY_DEV bool intersect_shape(const DevScene& s, uint32_t li, const DevObject& ob, V3 o, V3 d, V3 dinv, const TRay& r,
+                             Best& b) {
+    const float* od = s.odata + ob.data;
+    float t;
+    bool hit;
+    if (ob.kind == K_RECT_LIGHT) {
+        hit = rect_t(od, ob.ts, r.time, o, d, dinv, b.t, (s.flags & PSY_SCENE_RECT_LIGHT_FIX) != 0u, &t);
+    } else {
+        V3 c; float rad;
+        sphere_at(od, ob.ts, ob.kind == K_SPHERE ? 4 : 7, r.time, &c, &rad);
+        hit = sphere_t(o, d, b.t, c, rad, &t);
+    }
+    if (!hit) return false;
+    b.t = t; b.inst = li; b.aux = 0.0f; b.u = 0.0f; b.v = 0.0f;
+    return r.occl;
+}
+
+// The same for a leaf of the main pass, which walks patches itself: with
+// the patch case left out, the traversal loop does not carry a second,
+// unreachable split-tree walk and its registers.  (With it, the object-ray
+// build spilled 44 scalar registers to vector lanes inside the loop, the
+// world-ray build 42; without it 0 and 10, and the heightfield render at
+// 1024x1024x16 and the 10,000-light one are 1-2 % faster.)
+PSY_DEV bool intersect_shape_leaf(const DevScene& s, uint32_t li, const DevInstance& I, const TRay& r, Best& b) {
+    const DevObject ob = s.obj[I.object];
+    V3 o = r.o, d = r.d, dinv = r.dinv;
+    if (I.xf_count > 0) {
+        const M44 x = m_lerp_seq(r.time, s.xf + I.xf_offset, I.xf_count);
+        o = m_pos(x, r.o);
+        d = m_dir(x, r.d);
+        dinv = divv(splat(1.0f), d);
+    }
+    return intersect_shape(s, li, ob, o, d, dinv, r, b);
+}
+
 template <bool WORLD, int DEEP>
 PSY_DEV bool intersect_leaf(const DevScene& s, uint32_t li, const DevInstance& I, const TRay& r,
                                                Best& b, DeepState& need_deep) {
     const DevObject ob = s.obj[I.object];
     V3 o = r.o, d = r.d, dinv = r.dinv;
     RayW w = r.w;
+    const bool patch = ob.kind == K_BILINEAR || ob.kind == K_BICUBIC;
     if (I.xf_count > 0) {
         const M44 x = m_lerp_seq(r.time, s.xf + I.xf_offset, I.xf_count);
         o = m_pos(x, r.o);
         d = m_dir(x, r.d);
         dinv = divv(splat(1.0f), d);
-        if (WORLD && (ob.kind == K_BILINEAR || ob.kind == K_BICUBIC))
+        if (WORLD && patch)
             w = ray_widths(o, d, m_dir(x, r.odx), m_dir(x, r.ody), m_dir(x, r.ddx), m_dir(x, r.ddy));
     }
-    const float* od = s.odata + ob.data;
-    float t;
-    switch (ob.kind) {
-        case K_BILINEAR:
-        case K_BICUBIC:
-            return dice_walk<DEEP>(s, ob, li, o, dinv, w, r.occl, b, need_deep);
-        case K_SPHERE: {
-            V3 c; float rad;
-            sphere_at(od, ob.ts, 4, r.time, &c, &rad);
-            if (sphere_t(o, d, b.t, c, rad, &t)) {
-                b.t = t; b.inst = li; b.aux = 0.0f; b.u = 0.0f; b.v = 0.0f;
-                return r.occl;
-            }
-            return false;
-        }
-        case K_SPHERE_LIGHT: {
-            V3 c; float rad;
-            sphere_at(od, ob.ts, 7, r.time, &c, &rad);
-            if (sphere_t(o, d, b.t, c, rad, &t)) {
-                b.t = t; b.inst = li; b.aux = 0.0f; b.u = 0.0f; b.v = 0.0f;
-                return r.occl;
-            }
-            return false;
-        }
-        case K_RECT_LIGHT:
-            if (rect_t(od, ob.ts, r.time, o, d, dinv, b.t, (s.flags & PSY_SCENE_RECT_LIGHT_FIX) != 0u, &t)) {
-                b.t = t; b.inst = li; b.aux = 0.0f; b.u = 0.0f; b.v = 0.0f;
-                return r.occl;
-            }
-            return false;
-        default:
-            return false;
-    }
+    if (patch) return dice_walk<DEEP>(s, ob, li, o, dinv, w, r.occl, b, need_deep);
+    return intersect_shape(s, li, ob, o, d, dinv, r, b);
 }
 
 // Latitude / longitude parameters of a sphere hit, computed once for the
@@ -1208,8 +1212,7 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
         L.state |= LANE_WALKING;
         return false;
     }
-    DeepState unused{false, 0, nullptr};
-    return intersect_leaf<WORLD, D_FLAG>(s, li, I, L.r, L.b, unused);
+    return intersect_shape_leaf(s, li, I, L.r, L.b);
 }
 
 // The lane's final hit (t, inst, u, v, aux) in place in L.b; true if the
