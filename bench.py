@@ -326,7 +326,8 @@ def subdivision_stream(args):
         reps += 1
     ora_extract_ms = (time.perf_counter() - t0) / reps * 1e3
     ctx = gpu.Context(0)
-    ctx.set_continuation(args.continuation)
+    if args.continuation is not None:
+        ctx.set_continuation(args.continuation)
     t0 = time.perf_counter()
     g = gpu.GpuScene(ctx, scene_py, dice_depth=args.dice_depth)
     torch.cuda.synchronize()
@@ -441,8 +442,9 @@ def main():
     ap.add_argument("--trace-mode", choices=("persistent", "plain"), default="plain",
                     help="main trace pass: persistent waves with lane refill, or one thread per ray")
     ap.add_argument("--refill", type=int, default=16, help="persistent mode: refill a wave once this many lanes idle")
-    ap.add_argument("--continuation", type=int, default=24,
-                    help="plain mode: a wave hands its rays to a follow-on launch once fewer than this many trace (0: never)")
+    ap.add_argument("--continuation", type=int, default=None,
+                    help="plain mode: a wave hands its rays to a follow-on launch once fewer than this many trace "
+                         "(0: never; default: the library's, 24 for object rays and never for world rays)")
     ap.add_argument("--blocks-per-cu", type=int, default=0, help="persistent mode: blocks per CU (0: occupancy)")
     ap.add_argument("--split", action="store_true",
                     help="also time the primary and the bounce half of the stream separately (stderr)")
@@ -481,7 +483,8 @@ def main():
 
     log("setting up heightfield scene")
     ctx = gpu.Context(0)
-    ctx.set_continuation(args.continuation)
+    if args.continuation is not None:
+        ctx.set_continuation(args.continuation)
     ctx.set_trace_mode(persistent=args.trace_mode == "persistent", refill_min=args.refill,
                        blocks_per_cu=args.blocks_per_cu)
     scene_py = configs.heightfield_scene()
@@ -593,7 +596,7 @@ def main():
             "leaf_instances": int(info.n_leaf_instances),
             "bytes_per_ray": BYTES_PER_RAY,
             "trace_mode": args.trace_mode,
-            "continuation_below": args.continuation,
+            "continuation_below": 24 if args.continuation is None else args.continuation,
         },
         "roofline": {
             "kernel": "k_trace<false, 16, false> + k_trace_cont<false, 16> (main pass, %.3f ms/call)" % main_avg,

@@ -250,8 +250,8 @@ int psy_ctx_destroy(psy_ctx* ctx);
 int psy_ctx_set_trace_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_per_cu);
 /* Main-pass traversal stack in LDS (no counterpart in the reference, whose
  * BitStack and node stack live in CPU memory): 16 entries (default, 5 waves
- * per SIMD) or 32 (2 waves per SIMD; fewer rays handed to the second pass
- * on deep hierarchies).  Results are identical. */
+ * per SIMD) or 32 (2 waves per SIMD).  A ray whose stack outgrows them keeps
+ * the rest in the context's scratch.  Results are identical. */
 int psy_ctx_set_trace_stack(psy_ctx* ctx, int entries);
 /* The trace's second pass (no counterpart in the reference, which splits
  * patches per ray batch without a cache): rays that the main pass hands on
@@ -265,9 +265,11 @@ int psy_ctx_set_second_pass(psy_ctx* ctx, uint32_t wide_min, int32_t budget);
 /* The main pass's continuations (no counterpart in the reference, whose
  * lanes are CPU threads): the rays of one 64-lane wave end after very
  * different numbers of node steps, so once fewer than `below` of a wave's
- * rays are still tracing (1..64, default 24), their traversal state goes
- * to a continuation buffer in the context's scratch and a follow-on launch
- * finishes them 64 to a wave; 0 turns it off.  Results are identical.
+ * rays are still tracing (1..64), their traversal state goes to a
+ * continuation buffer in the context's scratch and a follow-on launch
+ * finishes them 64 to a wave; 0 turns it off.  Unless set, psy_trace_rays
+ * continues below 24 and everything that traces world rays does not.
+ * Results are identical.
  * psy_trace_rays_static never continues. */
 int psy_ctx_set_continuation(psy_ctx* ctx, int below);
 /* Paths per wavefront chunk of psy_render (no counterpart in the reference,
@@ -315,8 +317,8 @@ int psy_ctx_set_render_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_p
 /* Steps per captured graph of PSY_RENDER_STREAM: even, 2..64 (default 4). */
 int psy_ctx_set_stream_steps(psy_ctx* ctx, int steps_per_graph);
 /* Rays of the latest trace call on this context that the main pass handed
- * to the second pass (split below the dice cache, or a BVH stack deeper
- * than the main pass keeps).  Synchronizes the device; for diagnostics. */
+ * to the second pass (split below the dice cache, or a direction the main
+ * pass does not take).  Synchronizes the device; for diagnostics. */
 int psy_ctx_retrace_count(psy_ctx* ctx, int64_t* out);
 /* Rays of the latest trace call (psy_trace_*, or the last step of a
  * psy_render on the caller's stream) that took the second pass, and those of them that ran out of

@@ -886,9 +886,9 @@ PSY_DEV bool trace_one(const DevScene& s, const float* __restrict__ rays, int64_
 // resume at a pending sibling) -- so the 64 lanes of a wave advance
 // independently instead of waiting at every BVH leaf for the longest
 // split-tree walk in the wave.  Rays that reach the bottom of the dice cache
-// with a node still to split, or whose BVH stack would outgrow the main
-// pass's MAIN_STACK entries, are handed to the second pass, which retraces
-// them with a stack sized for the scene's worst case.
+// with a node still to split are handed to the second pass.  A BVH stack
+// that outgrows the main pass's MAIN_STACK entries of LDS keeps its bottom
+// in the trace's scratch pool (stack_spill).
 // ---------------------------------------------------------------------------
 #ifndef PSY_MAIN_STACK
 #define PSY_MAIN_STACK 16
@@ -932,6 +932,9 @@ struct Lane {
     // (CHILD_EMPTY: pop the stack)
     int32_t next;
     int sp;
+    // bottom stack entries moved out of LDS, as a list of pool chunks, the
+    // latest first (DEEP_NONE: none)
+    uint32_t spill;
     uint32_t state;  // LANE_* bits
     // the split-tree nodes at the bottom of the dice cache that still need
     // splitting, as a list in the trace's deep-node pool (DEEP_NONE: empty);
@@ -944,11 +947,16 @@ constexpr uint32_t DEEP_NONE = 0xffffffffu;
 // The deep-node pool of one trace call: entry e is 3 words (leaf instance,
 // heap node, next entry of the same ray's list or DEEP_NONE); `count` hands
 // out entries, `cap` bounds them (0: no pool, every such ray is retraced).
+// A chunk of SPILL_POOL consecutive entries holds SPILL_STACK entries of one
+// lane's traversal stack (ref and near distance each) and the link to the
+// lane's previous chunk.
 struct DeepPool {
     uint32_t* e;
     uint32_t* count;
     uint32_t cap;
 };
+constexpr int SPILL_STACK = 8;
+constexpr uint32_t SPILL_POOL = (2 * SPILL_STACK + 1 + 2) / 3;
 
 PSY_DEV uint32_t atomic_add_u32(uint32_t* p, uint32_t v) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -976,6 +984,46 @@ PSY_DEV uint32_t wave_alloc(uint32_t* counter, uint32_t want) {
 #else
     return __atomic_fetch_add(counter, want, __ATOMIC_RELAXED);
 #endif
+}
+
+// The lane's LDS stack is full: moves its SPILL_STACK bottom entries, which
+// are needed last, to a chunk of the pool; false when the pool has no room.
+// Rays whose stack outgrows LDS are few (300 of the 1.2 M rays of the
+// instanced, moving bicubic scene at 960x540x8), but handing them to the
+// second pass meant retracing each from the root, one to a wave, at the end
+// of the call: about 1 ms of latency per step.  That render went from 33.2
+// to 19.0 ms (with world rays no longer continued), one frame of its camera
+// rays at 960x540 from 1.27 to 0.76 ms.
+PSY_DEV bool stack_spill(Lane& L, int32_t (*stk_ref)[TRACE_BLOCK], float (*stk_near)[TRACE_BLOCK], int tid,
+                         const DeepPool& P) {
+    if (P.cap < SPILL_POOL) return false;
+    const uint32_t e = atomic_add_u32(P.count, SPILL_POOL);
+    if (e > P.cap - SPILL_POOL) return false;
+    uint32_t* c = P.e + 3 * (size_t)e;
+    for (int j = 0; j < SPILL_STACK; ++j) {
+        c[2 * j] = (uint32_t)stk_ref[j][tid];
+        c[2 * j + 1] = f2u(stk_near[j][tid]);
+    }
+    c[2 * SPILL_STACK] = L.spill;
+    L.spill = e;
+    for (int j = SPILL_STACK; j < L.sp; ++j) {
+        stk_ref[j - SPILL_STACK][tid] = stk_ref[j][tid];
+        stk_near[j - SPILL_STACK][tid] = stk_near[j][tid];
+    }
+    L.sp -= SPILL_STACK;
+    return true;
+}
+
+// The LDS stack is empty: brings the latest chunk back.
+PSY_DEV void stack_unspill(Lane& L, int32_t (*stk_ref)[TRACE_BLOCK], float (*stk_near)[TRACE_BLOCK], int tid,
+                           const DeepPool& P) {
+    const uint32_t* c = P.e + 3 * (size_t)L.spill;
+    for (int j = 0; j < SPILL_STACK; ++j) {
+        stk_ref[j][tid] = (int32_t)c[2 * j];
+        stk_near[j][tid] = u2f(c[2 * j + 1]);
+    }
+    L.spill = c[2 * SPILL_STACK];
+    L.sp = SPILL_STACK;
 }
 
 template <bool WORLD>
@@ -1009,6 +1057,7 @@ PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i) {
     L.depth = 0;
     L.next = s.root;
     L.sp = 0;
+    L.spill = DEEP_NONE;
     L.state = 0;
     L.deep_head = DEEP_NONE;
     L.wframe = -1;  // read by world rays only
@@ -1142,7 +1191,10 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
         ref = L.next;
         L.next = CHILD_EMPTY;
     } else {
-        if (L.sp == 0) return true;
+        if (L.sp == 0) {
+            if (L.spill == DEEP_NONE) return true;
+            stack_unspill(L, stk_ref, stk_near, tid, P);
+        }
         --L.sp;
         ref = stk_ref[L.sp][tid];
         if (!(stk_near[L.sp][tid] < L.b.t)) return false;
@@ -1181,7 +1233,9 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
         cmpswap(k1, r1, k3, r3);
         cmpswap(k1, r1, k2, r2);
         const int npush = (k1 < INFINITY ? 1 : 0) + (k2 < INFINITY ? 1 : 0) + (k3 < INFINITY ? 1 : 0);
-        if (L.sp + npush > STACK) {
+        // a scene without patches hands such a ray to the second pass, where
+        // a few nodes and shapes are soon retraced
+        if (L.sp + npush > STACK && !(s.dice && stack_spill(L, stk_ref, stk_near, tid, P))) {
             L.state |= LANE_RETRACE;
             return true;
         }
@@ -1296,8 +1350,8 @@ PSY_DEV void cont_save(uint32_t* __restrict__ cont, uint32_t cap, uint32_t e, co
     c[7 * m] = L.winst;
     c[8 * m] = L.k;
     c[9 * m] = L.trail;
-    c[10 * m] = (uint32_t)L.levels;
-    c[11 * m] = (uint32_t)L.depth;
+    c[10 * m] = (uint32_t)L.levels | (uint32_t)(L.depth + 1) << 8;
+    c[11 * m] = L.spill;
     c[12 * m] = (uint32_t)L.next;
     c[13 * m] = (uint32_t)L.sp;
     c[14 * m] = L.state;
@@ -1324,8 +1378,9 @@ PSY_DEV void cont_load(const DevScene& s, const float* __restrict__ rays, int64_
     L.winst = c[7 * m];
     L.k = c[8 * m];
     L.trail = c[9 * m];
-    L.levels = (int)c[10 * m];
-    L.depth = (int)c[11 * m];
+    L.levels = (int)(c[10 * m] & 0xffu);
+    L.depth = (int)(c[10 * m] >> 8) - 1;
+    L.spill = c[11 * m];
     L.next = (int32_t)c[12 * m];
     L.sp = (int)c[13 * m];
     L.state = c[14 * m];
