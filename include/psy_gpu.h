@@ -255,12 +255,11 @@ int psy_ctx_set_trace_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_pe
 int psy_ctx_set_trace_stack(psy_ctx* ctx, int entries);
 /* The trace's second pass (no counterpart in the reference, which splits
  * patches per ray batch without a cache): rays that the main pass hands on
- * are retraced one lane each, by a narrow build (1 wave per SIMD) for short
- * queues or a wide build (2 waves per SIMD) for queues of wide_min rays or
- * more (default 4096; 0: always the wide build; UINT32_MAX: always the
- * narrow one); a ray that takes more than `budget` (>= 1, default 512)
- * split-tree node expansions there goes on to the third, wave-cooperative
- * pass.  Results do not depend on either setting. */
+ * are worked one to a wave in short queues, or one to a lane in queues of
+ * wide_min rays or more (default 1024; 0: always a lane each; UINT32_MAX:
+ * always a wave each); a lane's ray that takes more than `budget` (>= 1,
+ * default 512) split-tree node expansions, or many cache nodes, goes on to
+ * the third pass, a wave each.  Results do not depend on either setting. */
 int psy_ctx_set_second_pass(psy_ctx* ctx, uint32_t wide_min, int32_t budget);
 /* The main pass's continuations (no counterpart in the reference, whose
  * lanes are CPU threads): the rays of one 64-lane wave end after very

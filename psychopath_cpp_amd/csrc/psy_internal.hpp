@@ -91,7 +91,7 @@ struct psy_ctx {
     bool scratch_recorded = false;
     // the allocation-free trace's scratch on this device (static_scratch_address)
     uint32_t* static_scratch = nullptr;
-    // second pass: queue length from which the wide build walks, node budget
+    // second pass: queue length from which it works a lane per ray, node budget
     uint32_t deep_wide_min = psy::DEEP_WIDE_MIN;
     int32_t deep_budget = psy::DEEP_BUDGET;
     // main-pass launch form, per ray form (0: object rays, 1: world rays)

@@ -179,8 +179,10 @@ __global__ __launch_bounds__(TRACE_BLOCK, persist_waves(WORLD, STACK)) void k_tr
     }
 }
 
-template <bool WORLD, int STACK, bool WIDE>
-__global__ __launch_bounds__(TRACE_BLOCK, WIDE ? DEEP_WIDE_WAVES : 1)
+// Second pass over a queue of wide_min rays or more, a lane per ray, within a
+// node budget per ray.
+template <bool WORLD, int STACK>
+__global__ __launch_bounds__(TRACE_BLOCK, DEEP_WIDE_WAVES)
 void k_trace_deep(DevScene s, const float* __restrict__ rays, int64_t n, int64_t rs, DevHits h, uint32_t flags,
                   const uint32_t* __restrict__ queue, const uint32_t* __restrict__ heads,
                   const uint32_t* __restrict__ pool, uint32_t* __restrict__ counters,
@@ -189,10 +191,10 @@ void k_trace_deep(DevScene s, const float* __restrict__ rays, int64_t n, int64_t
     __shared__ float stk_near[STACK][TRACE_BLOCK];
     const int tid = threadIdx.x;
     const uint32_t count = counters[0];
-    if (WIDE != (count >= wide_min)) return;  // the other build walks this queue
-    // Queue entry k goes to wave k % n_waves, lane k / n_waves: a short queue
-    // puts one ray in each wave, so rays that take different paths through
-    // the split trees run side by side instead of serializing in one wave.
+    if (count < wide_min) return;  // k_trace_coop works this queue
+    // Queue entry k goes to wave k % n_waves, lane k / n_waves: the shorter
+    // the queue, the fewer rays, which take different paths through the
+    // split trees, serialize in one wave.
     const uint32_t n_waves = gridDim.x * (TRACE_BLOCK / 64);
     const uint32_t wave = blockIdx.x * (TRACE_BLOCK / 64) + (uint32_t)(tid >> 6);
     const uint32_t lane = (uint32_t)(tid & 63);
@@ -200,37 +202,50 @@ void k_trace_deep(DevScene s, const float* __restrict__ rays, int64_t n, int64_t
         const uint32_t e = queue[k];
         const uint32_t i = e & ~QUEUE_RESUME;
         if ((int64_t)i >= n) continue;  // entries are ray indices of this call
-        // a ray that runs out of node budget goes to the third pass
+        // a ray that runs out of node budget goes to the third pass, by its queue entry
         bool more;
         if (e & QUEUE_RESUME) {
             more = resume_list<WORLD>(s, rays, rs, (int64_t)i, heads[k], pool, h, flags, budget);
         } else {
             more = trace_one<WORLD, STACK, D_SERIAL>(s, rays, rs, (int64_t)i, h, flags, stk_ref, stk_near, tid, budget);
         }
-        if (more) coop_queue[atomicAdd(&counters[1], 1u)] = i;
+        if (more) coop_queue[atomicAdd(&counters[1], 1u)] = (uint32_t)k;
     }
 }
 
-// Third pass: the rays whose split trees outran the second pass's budget,
-// one per wave, every lane of the wave on the same ray; the split-dice
-// below the cache runs across the lanes from a node stack in LDS.
+// One ray per wave, every lane of the wave on the same ray: the second pass
+// over a queue shorter than wide_min, or the third pass, over the rays whose
+// split trees outran k_trace_deep's budget.  The nodes on a ray's list are
+// shared out among the lanes, and the split-dice below one node runs across
+// the lanes from a node stack in LDS.
 template <bool WORLD, int STACK>
 __global__ __launch_bounds__(TRACE_BLOCK) void k_trace_coop(DevScene s, const float* __restrict__ rays, int64_t n,
                                                              int64_t rs, DevHits h, uint32_t flags,
+                                                             const uint32_t* __restrict__ queue,
+                                                             const uint32_t* __restrict__ heads,
+                                                             const uint32_t* __restrict__ pool,
                                                              const uint32_t* __restrict__ counters,
-                                                             const uint32_t* __restrict__ coop_queue) {
+                                                             const uint32_t* __restrict__ coop_queue,
+                                                             uint32_t wide_min) {
     __shared__ int32_t stk_ref[STACK][TRACE_BLOCK];
     __shared__ float stk_near[STACK][TRACE_BLOCK];
     __shared__ uint64_t nodes[TRACE_BLOCK / 64][COOP_CAP];
     const int tid = threadIdx.x;
-    const uint32_t count = counters[1];
+    const bool second = counters[0] < wide_min;
+    const uint32_t count = second ? counters[0] : counters[1];
     const uint32_t n_waves = gridDim.x * (TRACE_BLOCK / 64);
     const uint32_t wib = (uint32_t)(tid >> 6);
     for (uint32_t k = blockIdx.x * (TRACE_BLOCK / 64) + wib; k < count; k += n_waves) {
-        const uint32_t i = coop_queue[k];  // wave-uniform
+        const uint32_t slot = second ? k : coop_queue[k];  // wave-uniform
+        if ((int64_t)slot >= n) continue;
+        const uint32_t e = queue[slot];
+        const uint32_t i = e & ~QUEUE_RESUME;
         if ((int64_t)i >= n) continue;
-        (void)trace_one<WORLD, STACK, D_COOP>(s, rays, rs, (int64_t)i, h, flags, stk_ref, stk_near, tid, INT32_MAX,
-                                              nodes[wib]);
+        if (e & QUEUE_RESUME)
+            resume_list_coop<WORLD>(s, rays, rs, (int64_t)i, heads[slot], pool, h, flags, nodes[wib]);
+        else
+            (void)trace_one<WORLD, STACK, D_COOP>(s, rays, rs, (int64_t)i, h, flags, stk_ref, stk_near, tid, INT32_MAX,
+                                                  nodes[wib]);
     }
 }
 
@@ -757,19 +772,17 @@ template <bool W, int S>
 static void launch_deep(const DevScene& s, const float* rays, int64_t n, int64_t rs, const DevHits& h, uint32_t flags,
                         const uint32_t* queue, const uint32_t* heads, const uint32_t* pool, uint32_t* counters,
                         const TraceTuning& tune, hipStream_t st) {
-    const unsigned blocks = (unsigned)std::min<int64_t>(grid_for(n, TRACE_BLOCK), DEEP_ROUND);
+    // a wave per ray, of which a call hands on few
+    const unsigned blocks = (unsigned)std::min<int64_t>((n + 7) / 8, DEEP_ROUND);
     uint32_t* coop_queue = const_cast<uint32_t*>(queue) + n;
     const int32_t budget = std::max<int32_t>(1, tune.deep_budget);
-    if (tune.wide_min > 0)
-        hipLaunchKernelGGL((k_trace_deep<W, S, false>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, s, rays, n, rs, h,
-                           flags, queue, heads, pool, counters, coop_queue, tune.wide_min, budget);
     if (n >= (int64_t)tune.wide_min) {
         const unsigned wide = (unsigned)std::min<int64_t>(grid_for(n, TRACE_BLOCK), DEEP_ROUND * DEEP_WIDE_WAVES);
-        hipLaunchKernelGGL((k_trace_deep<W, S, true>), dim3(wide), dim3(TRACE_BLOCK), 0, st, s, rays, n, rs, h,
+        hipLaunchKernelGGL((k_trace_deep<W, S>), dim3(wide), dim3(TRACE_BLOCK), 0, st, s, rays, n, rs, h,
                            flags, queue, heads, pool, counters, coop_queue, tune.wide_min, budget);
     }
     hipLaunchKernelGGL((k_trace_coop<W, S>), dim3(blocks), dim3(TRACE_BLOCK), 0, st, s, rays, n, rs, h, flags,
-                       (const uint32_t*)counters, (const uint32_t*)coop_queue);
+                       queue, heads, pool, (const uint32_t*)counters, (const uint32_t*)coop_queue, tune.wide_min);
 }
 
 // The main pass one thread per ray, then the rays it continued (when the

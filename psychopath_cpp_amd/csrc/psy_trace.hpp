@@ -191,8 +191,10 @@ constexpr int COOP_CAP = 2048;         // node stack entries per wave in the thi
 // graze a surface: their slab overlaps long runs of micro-bboxes, and a
 // fixed order can improve the hit at every one of them, while near-to-far
 // prunes all but the first.  The walk keeps no patch stack: a node is its
-// path of halves (`pb`, deepest half in bit 0), replayed from `base`, and
-// `trail` has one bit per depth whose sibling is pending.  The reference's
+// path of halves (`pb`, deepest half in bit 0), and `trail` has one bit per
+// depth whose sibling is pending.  On the way down the current node's patch
+// stays in registers; only a pending sibling is replayed from `base`
+// (replaying every node made the walk's length quadratic in its depth).  The reference's
 // split-stack index (object/patch_utils.hpp:80: a node at index 63 is a
 // leaf) grows by one for every second half on the path.
 template <int N>
@@ -201,16 +203,15 @@ PSY_DEV bool dice_deep_from(const DevScene& s, const Patch<N>& base, const float
     int k = 0;           // depth below the start node
     uint64_t pb = 0;     // path of the current node
     uint64_t trail = 0;  // bit d: the sibling of the path's node at depth d is pending
-    bool expand = true;  // the current node is hit and needs splitting
+    bool expand = true;  // the current node (p, uv) is hit and needs splitting
+    Patch<N> p = base;
+    float uv[4] = {uvb[0], uvb[1], uvb[2], uvb[3]};
     for (;;) {
         if (expand) {
             if (--ds.budget < 0) {
                 ds.need = true;
                 return true;
             }
-            Patch<N> p = base;
-            float uv[4] = {uvb[0], uvb[1], uvb[2], uvb[3]};
-            for (int l = k - 1; l >= 0; --l) patch_step<N>(p, ((pb >> l) & 1ull) != 0, uv);
             Patch<N> p1 = p;
             float uv1[4] = {uv[0], uv[1], uv[2], uv[3]};
             patch_step<N>(p1, true, uv1);
@@ -257,6 +258,10 @@ PSY_DEV bool dice_deep_from(const DevScene& s, const Patch<N>& base, const float
                 if (go0 && go1) trail |= 1ull << (k + 1);
                 pb = (pb << 1) | (take1 ? 1ull : 0ull);
                 ++k;
+                if (take1) {
+                    p = p1;
+                    for (int j = 0; j < 4; ++j) uv[j] = uv1[j];
+                }
                 continue;
             }
         }
@@ -266,8 +271,8 @@ PSY_DEV bool dice_deep_from(const DevScene& s, const Patch<N>& base, const float
         trail &= ~(1ull << d);
         pb = (pb >> (k - d)) ^ 1ull;
         k = d;
-        Patch<N> p = base;
-        float uv[4] = {uvb[0], uvb[1], uvb[2], uvb[3]};
+        p = base;
+        for (int j = 0; j < 4; ++j) uv[j] = uvb[j];
         for (int l = k - 1; l >= 0; --l) patch_step<N>(p, ((pb >> l) & 1ull) != 0, uv);
         V3 lo, hi;
         patch_bound<N>(p, &lo, &hi);
@@ -329,12 +334,13 @@ __device__ void coop_node_patch(const Patch<N>& base, const float uvb[4], uint64
 }
 
 // dice_deep with the 64 lanes of a wave on one ray (every lane calls it with
-// the same arguments): each round the lanes take up to 64 nodes off the
-// wave's LDS stack, split them, test both halves against the wave's best
-// hit, accept leaves and push the halves that need splitting (the nearer
-// one last, so it comes off first).  The closest hit is the same in any
-// visit order.  A half that finds the stack full is walked by its lane
-// alone.  Every lane returns the same result.
+// the same arguments): each round the idle lanes take nodes off the wave's
+// LDS stack, every lane with a node splits it, tests both halves against the
+// wave's best hit, accepts leaves, goes on with the nearer half that needs
+// splitting (kept in registers: only a node off the stack is replayed from
+// the base) and pushes the other.  The closest hit is the same in any visit
+// order.  A half that finds the stack full is walked by its lane alone.
+// Every lane returns the same result.
 template <int N>
 __device__ bool dice_deep_coop(const DevScene& s, const DevObject& ob, uint32_t k0, uint32_t inst, V3 o, V3 dinv,
                             const RayW& w, bool occl, Best& b, uint64_t* stk) {
@@ -345,29 +351,36 @@ __device__ bool dice_deep_coop(const DevScene& s, const DevObject& ob, uint32_t 
     const int sidx0 = __builtin_popcount(k0) - 1;
     const uint32_t lane = __lane_id();
     const unsigned long long lt = (1ull << lane) - 1ull;
-    if (lane == 0) stk[0] = 1ull;  // k0 itself
-    wave_lds_sync();
-    int count = 1;
-    while (count > 0) {
-        const int take = count < 64 ? count : 64;
-        const int base_i = count - take;
-        const bool active = (int)lane < take;
-        const uint64_t node = active ? stk[base_i + (int)lane] : 1ull;
-        count = base_i;
-        wave_lds_sync();
-        bool push0 = false, push1 = false, accepted = false;
-        uint64_t c0 = 0, c1 = 0;
-        uint64_t lower = 0, upper = 0;  // with both halves: the farther below, the nearer on top
-        if (active) {
+    int count = 0;             // stack entries (wave-uniform)
+    bool have = lane == 0;     // this lane holds a node to split: its path, patch and rectangle
+    uint64_t node = 1ull;      // k0 itself
+    Patch<N> p = base;
+    float uv[4] = {uvb[0], uvb[1], uvb[2], uvb[3]};
+    for (;;) {
+        const unsigned long long idle = __ballot(!have);
+        if (count > 0) {
+            const int take = min(count, __popcll(idle));
+            const int rank = __popcll(idle & lt);
+            if (!have && rank < take) {
+                node = stk[count - 1 - rank];
+                have = true;
+                coop_node_patch<N>(base, uvb, node, p, uv);
+            }
+            count -= take;
+            wave_lds_sync();
+        } else if (~idle == 0ull) {
+            return false;
+        }
+        bool push = false, accepted = false;
+        uint64_t far = 0;
+        if (have) {
             const int k = 63 - __builtin_clzll(node);
-            Patch<N> p;
-            float uv[4];
-            coop_node_patch<N>(base, uvb, node, p, uv);
             Patch<N> p1 = p;
             float uv1[4] = {uv[0], uv[1], uv[2], uv[3]};
             patch_step<N>(p1, true, uv1);
             patch_step<N>(p, false, uv);
             const int sidx = sidx0 + __builtin_popcountll(node) - 1;
+            bool go0 = false, go1 = false;
             float n0 = 0.0f, n1 = 0.0f;
             {
                 V3 lo, hi;
@@ -380,9 +393,8 @@ __device__ bool dice_deep_coop(const DevScene& s, const DevObject& ob, uint32_t 
                         accepted |= accept_leaf(h0, h1, (uv1[0] + uv1[1]) * 0.5f, (uv1[2] + uv1[3]) * 0.5f, max_dim,
                                                 inst, b);
                     } else {
-                        push1 = true;
+                        go1 = true;
                         n1 = h0;
-                        c1 = (node << 1) | 1ull;
                     }
                 }
             }
@@ -397,56 +409,41 @@ __device__ bool dice_deep_coop(const DevScene& s, const DevObject& ob, uint32_t 
                         accepted |= accept_leaf(h0, h1, (uv[0] + uv[1]) * 0.5f, (uv[2] + uv[3]) * 0.5f, max_dim,
                                                 inst, b);
                     } else {
-                        push0 = true;
+                        go0 = true;
                         n0 = h0;
-                        c0 = node << 1;
                     }
                 }
             }
             // the second half counts as nearer on ties
-            if (push0 && push1) {
-                const bool second_nearer = n1 <= n0;
-                lower = second_nearer ? c0 : c1;
-                upper = second_nearer ? c1 : c0;
-            } else {
-                lower = push0 ? c0 : c1;
+            const bool take1 = go1 && (!go0 || n1 <= n0);
+            push = go0 && go1;
+            have = go0 || go1;
+            far = (node << 1) | (take1 ? 0ull : 1ull);
+            node = (node << 1) | (take1 ? 1ull : 0ull);
+            if (take1) {
+                p = p1;
+                for (int j = 0; j < 4; ++j) uv[j] = uv1[j];
             }
         }
-        const bool pa = push0 || push1;
-        const bool pd = push0 && push1;
-        const unsigned long long ma = __ballot(pa), md = __ballot(pd);
-        const int na = __popcll(ma);
-        const int ia = count + __popcll(ma & lt);
-        const int ib = count + na + __popcll(md & lt);
-        DeepState solo{false, INT32_MAX, nullptr};
-        if (pa) {
-            if (ia < COOP_CAP) {
-                stk[ia] = lower;
+        const unsigned long long m = __ballot(push);
+        const int at = count + __popcll(m & lt);
+        if (push) {
+            if (at < COOP_CAP) {
+                stk[at] = far;
             } else {
+                DeepState solo{false, INT32_MAX, nullptr};
                 Patch<N> q;
                 float uq[4];
-                coop_node_patch<N>(base, uvb, lower, q, uq);
-                accepted |= dice_deep_from<N>(s, q, uq, sidx0 + __builtin_popcountll(lower) - 1, inst, o, dinv, w,
+                coop_node_patch<N>(base, uvb, far, q, uq);
+                accepted |= dice_deep_from<N>(s, q, uq, sidx0 + __builtin_popcountll(far) - 1, inst, o, dinv, w,
                                               occl, b, solo);
             }
         }
-        if (pd) {
-            if (ib < COOP_CAP) {
-                stk[ib] = upper;
-            } else {
-                Patch<N> q;
-                float uq[4];
-                coop_node_patch<N>(base, uvb, upper, q, uq);
-                accepted |= dice_deep_from<N>(s, q, uq, sidx0 + __builtin_popcountll(upper) - 1, inst, o, dinv, w,
-                                              occl, b, solo);
-            }
-        }
-        count = min(count + na + __popcll(md), COOP_CAP);
+        count = min(count + __popcll(m), COOP_CAP);
         wave_lds_sync();
         wave_best(b);
         if (occl && __ballot(accepted) != 0ull) return true;
     }
-    return false;
 }
 
 template <int DEEP>
@@ -748,16 +745,19 @@ PSY_DEV void cmpswap(float& ka, int32_t& ra, float& kb, int32_t& rb) {
 #define PSY_TRACE_BLOCK 64
 #endif
 constexpr int TRACE_BLOCK = PSY_TRACE_BLOCK;  // threads per block of the trace kernels
-// The second pass has two builds, both launched on every trace; each reads
-// the queue length and only one of them walks the queue.  The narrow one
-// runs 1 wave per SIMD (256 VGPRs, no spills): the lowest latency per ray,
-// for short queues (a primary stream hands on a few hundred rays).  The wide
-// one runs 2 waves per SIMD (128 VGPRs, paid for with spills): 1.4x the
-// throughput on long queues (a ground plane diced below the cache hands on
-// half the camera rays).  Each launches one resident round of 64-thread
-// blocks over 256 CUs, as does the third pass (1 wave per SIMD).  The
-// queue length that picks the wide build (DEEP_WIDE_MIN by default) and
-// the second pass's node budget (DEEP_BUDGET) are launch parameters.
+// The second pass comes in two forms, and each reads the queue length to
+// know which of them works the queue.  Below wide_min rays a wave takes one
+// ray with all its lanes (k_trace_coop, 1 wave per SIMD): the lowest latency
+// for the few rays a primary stream hands on.  Longer queues are worked a
+// lane per ray (k_trace_deep, 2 waves per SIMD: 256 VGPRs, paid for with
+// spills), and k_trace_coop follows as the third pass, over the rays that
+// outran a lane's limits.  wide_min is k_trace_coop's number of waves by
+// default, so that none of them takes one ray after another.  (Until it
+// worked on lists, short queues had a second build of k_trace_deep at 1 wave
+// per SIMD: the object stream of 2^22 rays is the same within 0.3 %, the
+// heightfield crop at 331x173x3, 8 calls of a few queued rays, 3.49 ms for
+// 3.65.)  Each form launches one resident round of 64-thread blocks over 256
+// CUs.  wide_min and the second pass's node budget are launch parameters.
 constexpr int DEEP_WIDE_WAVES = 2;
 constexpr int DEEP_ROUND = 1024;          // blocks per wave per SIMD over 256 CUs
 
@@ -1420,56 +1420,128 @@ PSY_DEV bool lane_run(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOCK
     }
 }
 
+// One cache node (leaf instance li, heap node k) that the main pass listed for
+// ray r: the split-dice below it, per DEEP, unless the node's cached box lies
+// beyond the hit found meanwhile.  Replaying a bicubic patch down to its node
+// takes some 15 splits, so that one test is cheap.  True when an occlusion
+// ray is done, or ds.need when the budget ran out.
+template <bool WORLD, int DEEP>
+PSY_DEV bool resume_node(const DevScene& s, const TRay& r, uint32_t li, uint32_t k, Best& b, DeepState& ds) {
+    const DevInstance I = s.inst[li];
+    const DevObject ob = s.obj[I.object];
+    V3 o = r.o, dinv = r.dinv;
+    RayW w = r.w;
+    if (I.xf_count > 0) {
+        const M44 x = m_lerp_seq(r.time, s.xf + I.xf_offset, I.xf_count);
+        o = m_pos(x, r.o);
+        const V3 d = m_dir(x, r.d);
+        dinv = divv(splat(1.0f), d);
+        if (WORLD) w = ray_widths(o, d, m_dir(x, r.odx), m_dir(x, r.ody), m_dir(x, r.ddx), m_dir(x, r.ddy));
+    }
+    const float4* q = s.dice + 2 * ob.dice + 2 * (size_t)k;
+    float h0, h1;
+    if (!patch_box_ray(xyz(q[0]), xyz(q[1]), o, dinv, b.t, &h0, &h1)) return false;
+    return deep_walk<DEEP>(s, ob, k, li, o, dinv, w, r.occl, b, ds);
+}
+
+// The hit the main pass wrote for a ray that goes on from its list.
+PSY_DEV Best resume_hit(const DevHits& h, int64_t i, float max_t) {
+    Best b;
+    b.inst = h.inst[i];
+    b.t = b.inst != 0xffffffffu ? h.t[i] : max_t;
+    b.u = h.u[i];
+    b.v = h.v[i];
+    b.aux = h.aux ? h.aux[i] : 0.0f;
+    return b;
+}
+PSY_DEV void resume_store(const DevHits& h, int64_t i, const Best& b) {
+    h.t[i] = b.t;
+    h.inst[i] = b.inst;
+    h.u[i] = b.u;
+    h.v[i] = b.v;
+    if (h.aux) h.aux[i] = b.aux;
+}
+
 // Second pass for a ray the main pass left with a list of cache nodes to
 // split further: its hit so far (as the main pass wrote it), then the
 // split-dice below each listed node within a shared budget of node
 // expansions.  The main pass explored everything else with the same or a
 // looser bound on t, so the result is the full trace's.  Returns true when
-// the budget ran out (the ray then takes the third pass, which retraces it
-// whole).
+// the budget ran out, or RESUME_NODES nodes were walked and the list is not
+// done (the ray then takes the third pass, which walks its list again): most
+// lists hold one or two nodes, but a ray that grazes many patches can have
+// hundreds, and one lane needs about 5 us to replay the patch of each.
+// Camera rays over the subdivision scene at 641x479 (15,772 of them in the
+// second pass, 210 with more than 8 nodes): 1.39 ms a call for 3.1.
+constexpr int RESUME_NODES = 8;
 template <bool WORLD>
 PSY_DEV bool resume_list(const DevScene& s, const float* __restrict__ rays, int64_t n, int64_t i, uint32_t head,
                          const uint32_t* __restrict__ pool, const DevHits& h, uint32_t flags, int32_t budget) {
     TRay r;
     float max_t;
     load_ray<WORLD>(rays, n, i, flags, r, max_t);
-    Best b;
-    b.inst = h.inst[i];
-    const bool hit = b.inst != 0xffffffffu;
-    b.t = hit ? h.t[i] : max_t;
-    b.u = h.u[i];
-    b.v = h.v[i];
-    b.aux = h.aux ? h.aux[i] : 0.0f;
+    Best b = resume_hit(h, i, max_t);
     const uint32_t before = b.inst;
     const float t_before = b.t;
     DeepState ds{false, budget, nullptr};
-    for (uint32_t e = head; e != DEEP_NONE; e = pool[3 * e + 2]) {
-        const uint32_t li = pool[3 * e], k = pool[3 * e + 1];
-        const DevInstance I = s.inst[li];
-        const DevObject ob = s.obj[I.object];
-        V3 o = r.o, dinv = r.dinv;
-        RayW w = r.w;
-        if (I.xf_count > 0) {
-            const M44 x = m_lerp_seq(r.time, s.xf + I.xf_offset, I.xf_count);
-            o = m_pos(x, r.o);
-            const V3 d = m_dir(x, r.d);
-            dinv = divv(splat(1.0f), d);
-            if (WORLD) w = ray_widths(o, d, m_dir(x, r.odx), m_dir(x, r.ody), m_dir(x, r.ddx), m_dir(x, r.ddy));
-        }
-        bool done;
-        if (ob.kind == K_BILINEAR) done = dice_deep<4>(s, ob, k, li, o, dinv, w, r.occl, b, ds);
-        else done = dice_deep<16>(s, ob, k, li, o, dinv, w, r.occl, b, ds);
+    int walked = 0;
+    for (uint32_t e = head; e != DEEP_NONE; e = pool[3 * (size_t)e + 2]) {
+        if (walked == RESUME_NODES) return true;
+        const int32_t left = ds.budget;
+        const bool done = resume_node<WORLD, D_SERIAL>(s, r, pool[3 * (size_t)e], pool[3 * (size_t)e + 1], b, ds);
         if (ds.need) return true;
         if (done) break;  // an occlusion ray found its hit
+        walked += ds.budget != left ? 1 : 0;
     }
-    if (b.inst != before || b.t != t_before) {
-        h.t[i] = b.t;
-        h.inst[i] = b.inst;
-        h.u[i] = b.u;
-        h.v[i] = b.v;
-        if (h.aux) h.aux[i] = b.aux;
-    }
+    if (b.inst != before || b.t != t_before) resume_store(h, i, b);
     return false;
+}
+
+// Third pass for such a ray, with the 64 lanes of a wave (every lane calls
+// it with the same arguments): the lanes take a listed node each, 64 at a
+// time, and the nodes that outrun a lane's budget are then split by all of
+// them together.  The rays that get here mostly do for the length of their
+// list (every node on it costs a replay of its patch from the root), which
+// 64 lanes shorten 64-fold.
+constexpr int32_t COOP_LANE_BUDGET = 64;
+template <bool WORLD>
+__device__ void resume_list_coop(const DevScene& s, const float* __restrict__ rays, int64_t n, int64_t i,
+                                 uint32_t head, const uint32_t* __restrict__ pool, const DevHits& h, uint32_t flags,
+                                 uint64_t* coop) {
+    TRay r;
+    float max_t;
+    load_ray<WORLD>(rays, n, i, flags, r, max_t);
+    Best b = resume_hit(h, i, max_t);
+    const uint32_t before = b.inst;
+    const float t_before = b.t;
+    const int lane = (int)__lane_id();
+    for (uint32_t e = head; e != DEEP_NONE;) {
+        uint32_t mine = DEEP_NONE;
+        for (int j = 0; j < 64 && e != DEEP_NONE; ++j) {
+            if (lane == j) mine = e;
+            e = pool[3 * (size_t)e + 2];
+        }
+        DeepState ds{false, COOP_LANE_BUDGET, nullptr};
+        uint32_t li = 0, k = 1;
+        bool done = false;
+        if (mine != DEEP_NONE) {
+            li = pool[3 * (size_t)mine];
+            k = pool[3 * (size_t)mine + 1];
+            done = resume_node<WORLD, D_SERIAL>(s, r, li, k, b, ds) && !ds.need;
+        }
+        wave_best(b);
+        if (__ballot(done) != 0ull) break;  // an occlusion ray found its hit
+        unsigned long long left = __ballot(ds.need);
+        for (; left != 0ull; left &= left - 1ull) {
+            const int l = __ffsll((long long)left) - 1;
+            DeepState all{false, INT32_MAX, coop};
+            if (resume_node<WORLD, D_COOP>(s, r, (uint32_t)__shfl((int)li, l), (uint32_t)__shfl((int)k, l), b, all)) {
+                e = DEEP_NONE;
+                break;
+            }
+        }
+    }
+    if (b.inst != before || b.t != t_before) resume_store(h, i, b);
 }
 
 // Main pass, one thread per ray.

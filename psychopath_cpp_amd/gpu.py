@@ -151,9 +151,9 @@ class Context:
         """psy_ctx_set_trace_stack: main-pass LDS stack entries (16 or 32)."""
         check(lib().psy_ctx_set_trace_stack(self.handle, int(entries)), "psy_ctx_set_trace_stack")
 
-    def set_second_pass(self, wide_min=4096, budget=512):
-        """psy_ctx_set_second_pass: queue length from which the second pass's wide build walks the queue
-        (0: always wide, 0xffffffff: always narrow) and its node budget per ray before the third pass."""
+    def set_second_pass(self, wide_min=1024, budget=512):
+        """psy_ctx_set_second_pass: queue length from which the second pass takes a lane per ray instead of a
+        wave (0: always, 0xffffffff: never) and its node budget per lane's ray before the third pass."""
         check(lib().psy_ctx_set_second_pass(self.handle, int(wide_min) & 0xFFFFFFFF, int(budget)),
               "psy_ctx_set_second_pass")
 
