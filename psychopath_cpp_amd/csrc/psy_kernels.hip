@@ -86,7 +86,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, main_waves(WORLD, STACK, COHERENT)) vo
         // fewer than cont.below lanes are still tracing, they are written
         // to the continuation buffer and finished by k_trace_cont, packed
         // 64 to a wave.
-        if (lane_run<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool, cont)) return;
+        if (lane_run<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool, cont, RayStream{rays, rs})) return;
     } else {
         bool done = false;
         for (;;) {
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, main_waves(WORLD, STACK, COHERENT)) vo
             if (busy == 0ull) break;
             const bool walk = !done && (L.state & LANE_WALKING) != 0;
             const bool walk_round = 2 * __popcll(__ballot(walk)) >= __popcll(busy);  // wave-uniform
-            if (!done && walk == walk_round && lane_step<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool))
+            if (!done && walk == walk_round && lane_step<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool, RayStream{rays, rs}))
                 done = true;
         }
     }
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, main_waves(WORLD, STACK)) void k_trace
     if (e >= count) return;
     Lane L;
     cont_load<WORLD, STACK>(s, rays, rs, flags, in.c, in.cap, e, L, stk_ref, stk_near, tid);
-    if (lane_run<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool, out)) return;
+    if (lane_run<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool, out, RayStream{rays, rs})) return;
     if (lane_finish(s, L, h)) enqueue_second(queue, heads, counters, L);
 }
 
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, persist_waves(WORLD, STACK)) void k_tr
             const bool walk_round = 2 * __popcll(__ballot(walk)) >= __popcll(busy);
             go = active && walk == walk_round;
         }
-        if (go && lane_step<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool)) {
+        if (go && lane_step<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool, RayStream{rays, rs})) {
             active = false;
             if (lane_finish(s, L, h)) enqueue_second(queue, heads, counters, L);
         }

@@ -1348,9 +1348,8 @@ PSY_DEV void lane_init_wray(const DevScene& s, const WRay& w, uint32_t i, Lane& 
     L.r.ddy = w.ddy;
     L.r.time = w.time;
     L.r.occl = w.type == PSY_RAY_OCCLUSION;
-    L.r.w = ray_widths(L.r.o, L.r.d, L.r.odx, L.r.ody, L.r.ddx, L.r.ddy);
     L.r.dinv = divv(splat(1.0f), L.r.d);
-    lane_start(s, L, L.r.occl ? 1.0f : INFINITY, i);
+    lane_start<true>(s, L, L.r.occl ? 1.0f : INFINITY, i);
 }
 
 // The ray a lane just traced, as a world ray.

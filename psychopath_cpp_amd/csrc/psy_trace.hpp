@@ -111,6 +111,27 @@ PSY_DEV void load_patch(const float* odata, int32_t off, Patch<N>& p) {
     for (int i = 0; i < N; ++i) p.p[i] = mk(odata[off + 3 * i], odata[off + 3 * i + 1], odata[off + 3 * i + 2]);
 }
 
+// A node's parameter rectangle is dyadic: it lies at (iu, iv) of a 2^nu by
+// 2^nv grid, with nu + nv its depth (at most 24).  Its centre is kept as one
+// word, nu above 25 bits of (1 << depth | iu << nv | iv), which leaves the
+// other spare word of the node for its longest side: every visit needs the
+// side, only the one hit that is reported needs the centre.
+PSY_DEV uint32_t uv_code(const float uv[4], int depth) {
+    const int nu = 127 - (int)(f2u(uv[1] - uv[0]) >> 23);
+    const int nv = depth - nu;
+    const uint32_t iu = (uint32_t)(uv[0] * (float)(1u << nu)), iv = (uint32_t)(uv[2] * (float)(1u << nv));
+    return (uint32_t)nu << 25 | 1u << depth | iu << nv | iv;
+}
+// The centre ((uv0 + uv1) / 2 per axis, as floats) of a uv_code.
+PSY_DEV void uv_decode(uint32_t code, float* u, float* v) {
+    const uint32_t m = code & 0x1ffffffu;
+    const int nu = (int)(code >> 25), depth = heap_depth(m), nv = depth - nu;
+    const uint32_t i = m ^ (1u << depth);
+    // 2 i + 1 has up to 25 bits: rounded as the sum of the two edges is
+    *u = (float)(2u * (i >> nv) + 1u) * u2f((uint32_t)(126 - nu) << 23);
+    *v = (float)(2u * (i & ((1u << nv) - 1u)) + 1u) * u2f((uint32_t)(126 - nv) << 23);
+}
+
 template <int N>
 PSY_DEV_FN void build_node(const float* odata, const DevObject& ob, uint32_t k, float4* out) {
     Patch<N> p;
@@ -119,8 +140,8 @@ PSY_DEV_FN void build_node(const float* odata, const DevObject& ob, uint32_t k, 
     patch_at_node<N>(p, k, uv);
     V3 lo, hi;
     patch_bound<N>(p, &lo, &hi);
-    out[0] = make_float4(lo.x, lo.y, lo.z, (uv[0] + uv[1]) * 0.5f);
-    out[1] = make_float4(hi.x, hi.y, hi.z, (uv[2] + uv[3]) * 0.5f);
+    out[0] = make_float4(lo.x, lo.y, lo.z, longest_axis(sub(hi, lo)));
+    out[1] = make_float4(hi.x, hi.y, hi.z, u2f(uv_code(uv, heap_depth(k))));
 }
 
 
@@ -149,6 +170,13 @@ PSY_DEV bool accept_leaf(float h0, float h1, float u, float v, float maxd, uint3
         return true;
     }
     return false;
+}
+
+// The same for a node of the dice cache: its longest side and uv_code.
+PSY_DEV bool accept_node(float h0, float h1, float maxd, float code, uint32_t inst, Best& b) {
+    if (!accept_leaf(h0, h1, 0.0f, 0.0f, maxd, inst, b)) return false;
+    uv_decode(f2u(code), &b.u, &b.v);
+    return true;
 }
 
 // bbox_ray for a box of a patch's split tree, taking a NaN far distance as a
@@ -473,9 +501,8 @@ PSY_DEV bool dice_walk(const DevScene& s, const DevObject& ob, uint32_t inst, V3
         const float4 a = nodes[2], c = nodes[3];
         float h0, h1;
         if (!patch_box_ray(xyz(a), xyz(c), o, dinv, b.t, &h0, &h1)) return false;
-        const float maxd = longest_axis(sub(xyz(c), xyz(a)));
-        if (maxd <= dice_width(min_width(w, h0, h1) * s.dice_rate, s.min_upoly))
-            return accept_leaf(h0, h1, a.w, c.w, maxd, inst, b) && occl;
+        if (a.w <= dice_width(min_width(w, h0, h1) * s.dice_rate, s.min_upoly))
+            return accept_node(h0, h1, a.w, c.w, inst, b) && occl;
         if (levels == 0) return deep_walk<DEEP>(s, ob, 1, inst, o, dinv, w, occl, b, need_deep);
     }
     uint32_t k = 1;
@@ -491,17 +518,15 @@ PSY_DEV bool dice_walk(const DevScene& s, const DevObject& ob, uint32_t inst, V3
         const bool hit1 = patch_box_ray(xyz(a1), xyz(e1), o, dinv, b.t, &h10, &h11);
         bool split0 = false, split1 = false;
         if (hit1) {
-            const float maxd = longest_axis(sub(xyz(e1), xyz(a1)));
-            if (maxd <= dice_width(min_width(w, h10, h11) * s.dice_rate, s.min_upoly)) {
-                if (accept_leaf(h10, h11, a1.w, e1.w, maxd, inst, b) && occl) return true;
+            if (a1.w <= dice_width(min_width(w, h10, h11) * s.dice_rate, s.min_upoly)) {
+                if (accept_node(h10, h11, a1.w, e1.w, inst, b) && occl) return true;
             } else {
                 split1 = true;
             }
         }
         if (hit0) {
-            const float maxd = longest_axis(sub(xyz(e0), xyz(a0)));
-            if (maxd <= dice_width(min_width(w, h00, h01) * s.dice_rate, s.min_upoly)) {
-                if (accept_leaf(h00, h01, a0.w, e0.w, maxd, inst, b) && occl) return true;
+            if (a0.w <= dice_width(min_width(w, h00, h01) * s.dice_rate, s.min_upoly)) {
+                if (accept_node(h00, h01, a0.w, e0.w, inst, b) && occl) return true;
             } else {
                 split0 = true;
             }
@@ -535,9 +560,8 @@ PSY_DEV bool dice_walk(const DevScene& s, const DevObject& ob, uint32_t inst, V3
             const float4 a = nodes[2 * k], c = nodes[2 * k + 1];
             float h0, h1;
             if (!patch_box_ray(xyz(a), xyz(c), o, dinv, b.t, &h0, &h1)) continue;
-            const float maxd = longest_axis(sub(xyz(c), xyz(a)));
-            if (maxd <= dice_width(min_width(w, h0, h1) * s.dice_rate, s.min_upoly)) {
-                if (accept_leaf(h0, h1, a.w, c.w, maxd, inst, b) && occl) return true;
+            if (a.w <= dice_width(min_width(w, h0, h1) * s.dice_rate, s.min_upoly)) {
+                if (accept_node(h0, h1, a.w, c.w, inst, b) && occl) return true;
                 continue;
             }
             break;
@@ -910,24 +934,29 @@ constexpr int main_waves(bool world, int stack, bool coherent = false) {
 #endif
 constexpr int persist_waves(bool world, int stack) { return stack <= 16 ? PSY_PERSIST_WAVES_PER_SIMD : 2; }
 
+// A ray footprint as the walk uses it: per axis the width at t is
+// |k + dw t| + fw, except fw on an interval that holds the flip distance
+// (min_width_flip, with k = ow - fw).
+struct Foot { float kx, ky, dwx, dwy, fwx, fwy, flx, fly; };
+
 struct Lane {
     TRay r;
-    Best b;
+    Best b;  // while tracing, a patch hit's u holds its uv_code
     uint32_t idx;
     // split-tree walk (valid while walking): the patch's dice-cache slot,
-    // the heap node k being expanded at `depth`, and one `trail` bit per
-    // depth whose other child is still to be expanded; world rays also keep
-    // the patch-space ray and footprint (object rays never meet transformed
-    // patches, so theirs is the ray itself)
+    // the heap node k being expanded, and one `trail` bit per depth whose
+    // other child is still to be expanded; world rays also keep the
+    // patch-space ray (object rays never meet transformed patches, so
+    // theirs is the ray itself)
     uint32_t slot;
     V3 wo, wdinv;
-    RayW ww;
-    float wfx, wfy;  // flip distances of the patch-space footprint
-    // the leaf transforms wo .. wfy were derived for: the first transform's
-    // index, -2 for an untransformed leaf, -1 for none yet
+    Foot foot;
+    // the leaf transforms wo .. foot were derived for: the first transform's
+    // index, -2 for an untransformed leaf, -1 for none yet (object rays
+    // derive theirs once, when they start)
     int32_t wframe;
     uint32_t winst, k, trail;
-    int levels, depth;
+    int levels;
     // BVH: the nearest hit child, visited next without a stack round trip
     // (CHILD_EMPTY: pop the stack)
     int32_t next;
@@ -1030,9 +1059,62 @@ template <bool WORLD>
 PSY_DEV V3 walk_o(const Lane& L) { return WORLD ? L.wo : L.r.o; }
 template <bool WORLD>
 PSY_DEV V3 walk_dinv(const Lane& L) { return WORLD ? L.wdinv : L.r.dinv; }
-template <bool WORLD>
-PSY_DEV const RayW& walk_w(const Lane& L) { return WORLD ? L.ww : L.r.w; }
 
+// Where a lane finds its world ray's direction and differentials, which it
+// needs only when it derives a patch-space ray: in the lane's registers, or
+// in the ray stream, which keeps 15 registers free during the traversal.
+struct RayRegs {
+    PSY_DEV void get(const Lane& L, V3* odx, V3* ody, V3* ddx, V3* ddy) const {
+        *odx = L.r.odx; *ody = L.r.ody; *ddx = L.r.ddx; *ddy = L.r.ddy;
+    }
+};
+struct RayStream {
+    const float* rays;
+    int64_t n;
+    PSY_DEV void get(const Lane& L, V3* odx, V3* ody, V3* ddx, V3* ddy) const {
+        uint32_t i = L.idx;
+#if defined(__HIP_DEVICE_COMPILE__)
+        // the twelve addresses are computed here, not ahead of the loop,
+        // where they would be held in registers
+        asm volatile("" : "+v"(i));
+#endif
+        const float* q = rays + i;
+        *odx = mk(q[6 * n], q[7 * n], q[8 * n]);
+        *ody = mk(q[9 * n], q[10 * n], q[11 * n]);
+        *ddx = mk(q[12 * n], q[13 * n], q[14 * n]);
+        *ddy = mk(q[15 * n], q[16 * n], q[17 * n]);
+    }
+};
+
+// The walk's form of a footprint; false for one with an infinite term, whose
+// widths can be NaN at some distances only (the second pass follows the
+// reference there).  A footprint that is NaN on an axis makes the width NaN,
+// which dices to min_upoly (dice_width), as a width of 0 does; std::min
+// passes a NaN on when x has it and ignores it in y.
+PSY_DEV bool make_foot(const RayW& w, Foot& f) {
+    f.kx = w.owx - w.fwx; f.dwx = w.dwx; f.fwx = w.fwx;
+    f.ky = w.owy - w.fwy; f.dwy = w.dwy; f.fwy = w.fwy;
+    f.flx = flip_x(w);
+    f.fly = flip_y(w);
+    const bool nan_x = w.owx != w.owx || w.dwx != w.dwx || w.fwx != w.fwx;
+    const bool nan_y = w.owy != w.owy || w.dwy != w.dwy || w.fwy != w.fwy;
+    if (nan_x) { f.kx = f.dwx = f.fwx = 0.0f; f.flx = INFINITY; }
+    if (nan_y) { f.ky = f.dwy = 0.0f; f.fwy = INFINITY; f.fly = INFINITY; }
+    return finite3(mk(f.kx, f.dwx, f.fwx)) && finite3(mk(f.ky, f.dwy, nan_y ? 0.0f : f.fwy));
+}
+
+// min_width_flip over a box's near and far distance for a make_foot footprint
+// and a box that is hit (near is finite and not below 0; a far distance of
+// infinity times a dw of 0 is ignored by fminf as by std::min).
+PSY_DEV float foot_width(const Foot& f, float h0, float h1) {
+    float wx = fminf(fabsf(f.kx + f.dwx * h0), fabsf(f.kx + f.dwx * h1)) + f.fwx;
+    float wy = fminf(fabsf(f.ky + f.dwy * h0), fabsf(f.ky + f.dwy * h1)) + f.fwy;
+    wx = h0 < f.flx && h1 > f.flx ? f.fwx : wx;
+    wy = h0 < f.fly && h1 > f.fly ? f.fwy : wy;
+    return smin(wx, wy);
+}
+
+template <bool WORLD>
 PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i);
 
 template <bool WORLD>
@@ -1040,10 +1122,11 @@ PSY_DEV void lane_init(const DevScene& s, const float* __restrict__ rays, int64_
                                           uint32_t flags, Lane& L) {
     float max_t;
     load_ray<WORLD>(rays, n, (int64_t)i, flags, L.r, max_t);
-    lane_start(s, L, max_t, i);
+    lane_start<WORLD>(s, L, max_t, i);
 }
 
 // Traversal state of a lane whose ray L.r is loaded.
+template <bool WORLD>
 PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i) {
     L.b.t = max_t;
     L.b.inst = 0xffffffffu;
@@ -1054,7 +1137,6 @@ PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i) {
     L.winst = 0;
     L.k = 0;
     L.trail = 0;
-    L.depth = 0;
     L.next = s.root;
     L.sp = 0;
     L.spill = DEEP_NONE;
@@ -1063,42 +1145,41 @@ PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i) {
     L.wframe = -1;  // read by world rays only
     // the main pass's box tests assume a finite inverse direction; the
     // second pass follows the reference's NaN behaviour exactly
-    if (!finite3(L.r.dinv)) {
+    bool plain = finite3(L.r.dinv);
+    if (!WORLD) plain = make_foot(L.r.w, L.foot) && plain;
+    if (!plain) {
         L.state = LANE_RETRACE;
         L.next = CHILD_EMPTY;
     }
 }
 
 // The patch-space ray of a walk through leaf I's split tree (world rays:
-// through the leaf's transform at the ray's time) and its footprint's flip
-// distances; false when its inverse direction is not finite.  They depend
+// through the leaf's transform at the ray's time) and its footprint; false
+// when its inverse direction or its footprint is not finite.  They depend
 // on the leaf's transforms alone, so the patches of one instance (a
 // subdivision surface's, an instanced assembly's) reuse them: a ray that
 // meets several patches of a transformed instance derives them once.
-template <bool WORLD>
-PSY_DEV bool walk_ray(const DevScene& s, Lane& L, const DevInstance& I) {
-    // object rays keep only the two flip distances, cheaper to re-derive
-    // than to hold in a register through the BVH walk
+template <class Src>
+PSY_DEV bool walk_ray(const DevScene& s, Lane& L, const DevInstance& I, const Src& src) {
     const int32_t frame = I.xf_count > 0 ? I.xf_offset : -2;
-    if (WORLD && frame == L.wframe) return true;
-    bool finite = true;
-    if (WORLD) {
-        L.wo = L.r.o;
-        L.wdinv = L.r.dinv;
-        L.ww = L.r.w;
-        if (I.xf_count > 0) {
-            const M44 x = m_lerp_seq(L.r.time, s.xf + I.xf_offset, I.xf_count);
-            L.wo = m_pos(x, L.r.o);
-            const V3 d = m_dir(x, L.r.d);
-            L.wdinv = divv(splat(1.0f), d);
-            finite = finite3(L.wdinv);
-            L.ww = ray_widths(L.wo, d, m_dir(x, L.r.odx), m_dir(x, L.r.ody), m_dir(x, L.r.ddx), m_dir(x, L.r.ddy));
-        }
+    if (frame == L.wframe) return true;
+    V3 odx, ody, ddx, ddy, d = L.r.d;
+    src.get(L, &odx, &ody, &ddx, &ddy);
+    L.wo = L.r.o;
+    L.wdinv = L.r.dinv;
+    if (I.xf_count > 0) {
+        const M44 x = m_lerp_seq(L.r.time, s.xf + I.xf_offset, I.xf_count);
+        L.wo = m_pos(x, L.wo);
+        d = m_dir(x, d);
+        L.wdinv = divv(splat(1.0f), d);
+        odx = m_dir(x, odx);
+        ody = m_dir(x, ody);
+        ddx = m_dir(x, ddx);
+        ddy = m_dir(x, ddy);
     }
-    L.wfx = flip_x(walk_w<WORLD>(L));
-    L.wfy = flip_y(walk_w<WORLD>(L));
-    if (WORLD) L.wframe = finite ? frame : -1;
-    return finite;
+    const bool plain = make_foot(ray_widths(L.wo, d, odx, ody, ddx, ddy), L.foot) && finite3(L.wdinv);
+    L.wframe = plain ? frame : -1;
+    return plain;
 }
 
 // One unit of work; true when the ray is finished (or must be retraced).
@@ -1109,78 +1190,74 @@ PSY_DEV bool walk_ray(const DevScene& s, Lane& L, const DevInstance& I) {
 //             box was already found hit and too large when its parent was
 //             expanded; its children lie inside it, so expanding it without
 //             a re-test finds the same hits)
-//   else    : one BVH4 node, or one leaf instance
-template <bool WORLD, int STACK = MAIN_STACK>
+//   else    : one BVH4 node, and the leaf instance that is nearest below it
+// A wave issues both kinds of step for whatever lanes need them, so the step
+// is written to issue little: the two children's tests and the choice
+// between them are straight-line selects, with branches only around what is
+// rare (a bottom node of the cache, a leaf).
+template <bool WORLD, int STACK = MAIN_STACK, class Src = RayRegs>
 PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOCK],
-                                          float (*stk_near)[TRACE_BLOCK], int tid, const DeepPool& P) {
+                                          float (*stk_near)[TRACE_BLOCK], int tid, const DeepPool& P,
+                                          const Src& src = Src()) {
     if (L.state & LANE_WALKING) {
         const uint32_t c0 = 2 * L.k;
         const float4* q = s.dice + 2 * ((size_t)L.slot + c0);
         const V3 wo = walk_o<WORLD>(L), wdinv = walk_dinv<WORLD>(L);
-        const RayW& ww = walk_w<WORLD>(L);
         const float4 a0 = q[0], e0 = q[1], a1 = q[2], e1 = q[3];
         float h00, h01, h10, h11;
         const bool hit0 = bbox_ray_fast(xyz(a0), xyz(e0), wo, wdinv, L.b.t, &h00, &h01) && L.k != 0;
         const bool hit1 = bbox_ray_fast(xyz(a1), xyz(e1), wo, wdinv, L.b.t, &h10, &h11);
-        bool split0 = false, split1 = false;
-        // the second half first: the reference visits it first on ties
-        if (hit1) {
-            const float maxd = longest_axis(sub(xyz(e1), xyz(a1)));
-            if (maxd <= dice_width(min_width_flip(ww, L.wfx, L.wfy, h10, h11) * s.dice_rate, s.min_upoly)) {
-                if (accept_leaf(h10, h11, a1.w, e1.w, maxd, L.winst, L.b) && L.r.occl) return true;
-            } else {
-                split1 = true;
-            }
-        }
-        if (hit0) {
-            const float maxd = longest_axis(sub(xyz(e0), xyz(a0)));
-            if (maxd <= dice_width(min_width_flip(ww, L.wfx, L.wfy, h00, h01) * s.dice_rate, s.min_upoly)) {
-                if (accept_leaf(h00, h01, a0.w, e0.w, maxd, L.winst, L.b) && L.r.occl) return true;
-            } else {
-                split0 = true;
-            }
-        }
-        split0 = split0 && h00 <= L.b.t;
-        split1 = split1 && h10 <= L.b.t;
-        const int cd = L.depth + 1;
-        if (cd == L.levels) {
+        // maxd <= dice_width(width), the maximum taken apart
+        const float w0 = foot_width(L.foot, h00, h01) * s.dice_rate;
+        const float w1 = foot_width(L.foot, h10, h11) * s.dice_rate;
+        const bool small0 = a0.w <= w0 || a0.w <= s.min_upoly;
+        const bool small1 = a1.w <= w1 || a1.w <= s.min_upoly;
+        // accept_leaf on both; the second half first, as the reference
+        // visits it first on ties (an occlusion ray takes the first it finds)
+        const float t0 = (h00 + h01) * 0.5f, t1 = (h10 + h11) * 0.5f;
+        const bool acc1 = hit1 && small1 && t1 > 0.0f && t1 < L.b.t;
+        if (acc1) { L.b.t = t1; L.b.inst = L.winst; L.b.u = e1.w; L.b.aux = a1.w; }
+        const bool acc0 = hit0 && small0 && t0 > 0.0f && t0 < L.b.t && !(acc1 && L.r.occl);
+        if (acc0) { L.b.t = t0; L.b.inst = L.winst; L.b.u = e0.w; L.b.aux = a0.w; }
+        if ((acc0 || acc1) && L.r.occl) return true;
+        bool split0 = hit0 && !small0 && h00 <= L.b.t;
+        bool split1 = hit1 && !small1 && h10 <= L.b.t;
+        const int cd = L.k ? 32 - __builtin_clz(L.k) : 0;  // the children's depth
+        if (cd == L.levels && (split0 || split1)) {
             // children that need splits below the cache go onto the lane's
             // list for the second pass to resume from
             const uint32_t nd = (split0 ? 1u : 0u) + (split1 ? 1u : 0u);
-            if (nd) {
-                L.state |= LANE_NEED_DEEP;
-                // rare, so one atomic per lane (a wave-aggregated one costs the main
-                // pass registers)
-                const uint32_t e0 = P.cap ? atomic_add_u32(P.count, nd) : 0u;
-                if (e0 + nd > P.cap) {
-                    L.state |= LANE_DEEP_MANY;
-                } else {
-                    uint32_t e = e0;
-                    if (split1) {
-                        P.e[3 * e] = L.winst; P.e[3 * e + 1] = c0 + 1; P.e[3 * e + 2] = L.deep_head;
-                        L.deep_head = e++;
-                    }
-                    if (split0) {
-                        P.e[3 * e] = L.winst; P.e[3 * e + 1] = c0; P.e[3 * e + 2] = L.deep_head;
-                        L.deep_head = e;
-                    }
+            L.state |= LANE_NEED_DEEP;
+            // rare, so one atomic per lane (a wave-aggregated one costs the main
+            // pass registers)
+            const uint32_t at = P.cap ? atomic_add_u32(P.count, nd) : 0u;
+            if (at + nd > P.cap) {
+                L.state |= LANE_DEEP_MANY;
+            } else {
+                uint32_t e = at;
+                if (split1) {
+                    uint32_t* w = P.e + 3 * (size_t)e;
+                    w[0] = L.winst; w[1] = c0 + 1; w[2] = L.deep_head;
+                    L.deep_head = e++;
+                }
+                if (split0) {
+                    uint32_t* w = P.e + 3 * (size_t)e;
+                    w[0] = L.winst; w[1] = c0; w[2] = L.deep_head;
+                    L.deep_head = e;
                 }
             }
             split0 = split1 = false;
         }
-        if (split0 && split1) {
-            L.k = (h00 < h10) ? c0 : c0 + 1;
-            L.trail |= 1u << cd;
-            L.depth = cd;
-        } else if (split0 || split1) {
-            L.k = split0 ? c0 : c0 + 1;
-            L.depth = cd;
+        if (split0 || split1) {
+            // the nearer child, the second on ties
+            const bool second = split1 && !(split0 && h00 < h10);
+            L.k = c0 + (second ? 1u : 0u);
+            L.trail |= split0 && split1 ? 1u << cd : 0u;
         } else if (L.trail == 0) {
             L.state &= ~LANE_WALKING;
         } else {
             const int dd = 31 - __builtin_clz(L.trail);
-            L.k = (L.k >> (L.depth - dd)) ^ 1u;
-            L.depth = dd;
+            L.k = (L.k >> (cd - 1 - dd)) ^ 1u;
             L.trail &= ~(1u << dd);
         }
         return false;
@@ -1242,8 +1319,12 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
         if (k3 < INFINITY) { stk_ref[L.sp][tid] = r3; stk_near[L.sp][tid] = k3; ++L.sp; }
         if (k2 < INFINITY) { stk_ref[L.sp][tid] = r2; stk_near[L.sp][tid] = k2; ++L.sp; }
         if (k1 < INFINITY) { stk_ref[L.sp][tid] = r1; stk_near[L.sp][tid] = k1; ++L.sp; }
-        if (k0 < INFINITY) L.next = r0;
-        return false;
+        if (!(k0 < INFINITY)) return false;
+        if (r0 >= 0) {
+            L.next = r0;
+            return false;
+        }
+        ref = r0;
     }
     // leaf instance: a patch starts a split-tree walk at its root
     const uint32_t li = (uint32_t)(~ref);
@@ -1257,9 +1338,8 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
         L.levels = I.dice_levels;
         L.winst = li;
         L.k = 0;
-        L.depth = -1;
         L.trail = 0;
-        if (!walk_ray<WORLD>(s, L, I)) {
+        if (WORLD && !walk_ray(s, L, I, src)) {
             L.state |= LANE_RETRACE;
             return true;
         }
@@ -1273,8 +1353,13 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
 // ray goes to the second pass.
 PSY_DEV bool lane_result(const DevScene& s, Lane& L) {
     const bool hit = L.b.inst != 0xffffffffu;
-    if (hit && !L.r.occl) sphere_uv(s, L.b, L.r);
-    if (!hit) L.b.t = INFINITY;
+    if (hit) {
+        const int32_t kind = s.inst[L.b.inst].kind;
+        if (kind == K_BILINEAR || kind == K_BICUBIC) uv_decode(f2u(L.b.u), &L.b.u, &L.b.v);
+        else if (!L.r.occl) sphere_uv(s, L.b, L.r);
+    } else {
+        L.b.t = INFINITY;
+    }
     return (L.state & (LANE_NEED_DEEP | LANE_RETRACE)) != 0 && !(L.r.occl && hit);
 }
 
@@ -1308,11 +1393,11 @@ PSY_DEV void enqueue_second(uint32_t* __restrict__ queue, uint32_t* __restrict__
 // continuation buffer and ends; a follow-on launch packs the continued
 // rays 64 to a wave and finishes them.  A lane's state is CONT_FIXED words
 // (best hit, ray index, walk state, BVH next / stack depth, flags, deep
-// list) plus its stack entries (ref, near); the ray itself is reloaded from
+// list, spilled stack) plus its stack entries (ref, near); the ray itself is reloaded from
 // the stream and its walk ray re-derived from the walked leaf, so each ray
 // takes the same steps as it would have in one launch.  Entry e's word w is
 // at cont[w * cap + e].
-constexpr int CONT_FIXED = 16;
+constexpr int CONT_FIXED = 15;
 // One level: the continued rays' own launch runs them to the end (a second
 // level, continuing that launch's tails again, was slower: 2.21 against
 // 2.01 ms on the 2^22-ray heightfield stream).
@@ -1343,19 +1428,18 @@ PSY_DEV void cont_save(uint32_t* __restrict__ cont, uint32_t cap, uint32_t e, co
     c[0 * m] = f2u(L.b.t);
     c[1 * m] = L.b.inst;
     c[2 * m] = f2u(L.b.u);
-    c[3 * m] = f2u(L.b.v);
+    c[3 * m] = L.spill;
     c[4 * m] = f2u(L.b.aux);
     c[5 * m] = L.idx;
     c[6 * m] = L.slot;
     c[7 * m] = L.winst;
     c[8 * m] = L.k;
     c[9 * m] = L.trail;
-    c[10 * m] = (uint32_t)L.levels | (uint32_t)(L.depth + 1) << 8;
-    c[11 * m] = L.spill;
+    c[10 * m] = (uint32_t)L.levels;
+    c[11 * m] = L.deep_head;
     c[12 * m] = (uint32_t)L.next;
     c[13 * m] = (uint32_t)L.sp;
     c[14 * m] = L.state;
-    c[15 * m] = L.deep_head;
     for (int j = 0; j < L.sp; ++j) {
         c[(CONT_FIXED + 2 * j) * m] = (uint32_t)stk_ref[j][tid];
         c[(CONT_FIXED + 2 * j + 1) * m] = f2u(stk_near[j][tid]);
@@ -1372,25 +1456,23 @@ PSY_DEV void cont_load(const DevScene& s, const float* __restrict__ rays, int64_
     L.b.t = u2f(c[0 * m]);
     L.b.inst = c[1 * m];
     L.b.u = u2f(c[2 * m]);
-    L.b.v = u2f(c[3 * m]);
+    L.spill = c[3 * m];
     L.b.aux = u2f(c[4 * m]);
     L.slot = c[6 * m];
     L.winst = c[7 * m];
     L.k = c[8 * m];
     L.trail = c[9 * m];
-    L.levels = (int)(c[10 * m] & 0xffu);
-    L.depth = (int)(c[10 * m] >> 8) - 1;
-    L.spill = c[11 * m];
+    L.levels = (int)c[10 * m];
+    L.deep_head = c[11 * m];
     L.next = (int32_t)c[12 * m];
     L.sp = (int)c[13 * m];
     L.state = c[14 * m];
-    L.deep_head = c[15 * m];
     for (int j = 0; j < L.sp; ++j) {
         stk_ref[j][tid] = (int32_t)c[(CONT_FIXED + 2 * j) * m];
         stk_near[j][tid] = u2f(c[(CONT_FIXED + 2 * j + 1) * m]);
     }
     // a walking lane's leaf gave a finite walk ray when the walk started
-    if (L.state & LANE_WALKING) (void)walk_ray<WORLD>(s, L, s.inst[L.winst]);
+    if (WORLD && (L.state & LANE_WALKING) != 0) (void)walk_ray(s, L, s.inst[L.winst], RayStream{rays, rs});
 }
 
 // Runs lane L to the end of its ray or, once fewer than `out.below` of the
@@ -1398,13 +1480,14 @@ PSY_DEV void cont_load(const DevScene& s, const float* __restrict__ rays, int64_
 // lanes together, if the buffer has room for them).  True when continued.
 template <bool WORLD, int STACK>
 PSY_DEV bool lane_run(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOCK],
-                      float (*stk_near)[TRACE_BLOCK], int tid, const DeepPool& pool, const ContBuf& out) {
+                      float (*stk_near)[TRACE_BLOCK], int tid, const DeepPool& pool, const ContBuf& out,
+                      const RayStream& src) {
     int below = out.below;  // wave-uniform
 #if !defined(__HIP_DEVICE_COMPILE__)
     (void)below;  // the host pass has no wave intrinsics
 #endif
     for (;;) {
-        if (lane_step<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool)) return false;
+        if (lane_step<WORLD, STACK>(s, L, stk_ref, stk_near, tid, pool, src)) return false;
 #if defined(__HIP_DEVICE_COMPILE__)
         const int live = __popcll(__ballot(1));
         if (live < below) {

@@ -1,0 +1,61 @@
+"""The dice cache's nodes (longest side and packed parameter centre) and the
+main pass's footprint test, on the CPU build of the device code: a cached
+walk gives what splitting the patch from its root gives (dice depth 0, where
+every split is the second pass's), to the bit."""
+import numpy as np
+import pytest
+
+from psychopath_cpp_amd import abi
+from psychopath_cpp_amd.scene import Assembly, Bicubic, Bilinear, Camera, Scene, look_at
+from tests.cpu_build import hostbuild
+
+
+def _scene(kind, min_upoly=1e-5):
+    root = Assembly()
+    sc = Scene(Camera([look_at((0, 0, 5), (0, 0, 0), (0, 1, 0))], [0.9]), root, dice_rate=1.0, min_upoly_size=min_upoly)
+    sc.add_surface_shader("s", abi.PSY_SHADER_LAMBERT, (0.5, 0.5, 0.5))
+    if kind == "long":  # splits u only for its first six levels
+        root.add_object("p", Bilinear([(-3, -0.05, 0), (3, -0.04, 0.3), (-3, 0.05, 0.1), (3, 0.06, 0.2)]))
+    elif kind == "bilinear":
+        root.add_object("p", Bilinear([(-1, -1, 0), (1, -1, 0.3), (-1, 1, 0.1), (1, 1, -0.2)]))
+    else:
+        rng = np.random.default_rng(3)
+        g = np.stack(np.meshgrid(np.linspace(-1, 1, 4), np.linspace(-1, 1, 4)), -1).reshape(16, 2)
+        root.add_object("p", Bicubic(np.concatenate([g, rng.uniform(-0.3, 0.3, (16, 1))], 1)))
+    root.create_object_instance("p", [], "s")
+    return sc
+
+
+def _object_rays(n, width):
+    rng = np.random.default_rng(5)
+    r = np.zeros((15, n), np.float32)
+    r[0:3] = rng.uniform(-0.3, 0.3, (3, n)) + np.array([[0], [0], [4.0]])
+    r[3:5] = rng.uniform(-0.3, 0.3, (2, n))
+    r[5] = -1.0
+    r[6] = np.inf
+    r[8:10] = width
+    return r
+
+
+@pytest.mark.parametrize("kind", ["long", "bilinear", "bicubic"])
+@pytest.mark.parametrize("depth,width", [(1, 0.2), (7, 0.03), (16, 0.004), (20, 0.002)])
+def test_cached_walk_equals_split_walk(kind, depth, width):
+    rays = _object_rays(600, width)
+    a = hostbuild.trace(_scene(kind), rays, world=False, dice_depth=depth)
+    b = hostbuild.trace(_scene(kind), rays, world=False, dice_depth=0)
+    assert (a["inst"] == 0).sum() > 20
+    for k in ("t", "inst", "u", "v", "aux"):
+        assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("plane", [8, 9, 10, 11, 12, 13])  # owx owy dwx dwy fwx fwy
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, 1e38])
+def test_footprints_that_are_not_finite(plane, value):
+    rays = _object_rays(60, 0.05)
+    rays[10:12] = 0.01
+    rays[plane] = value
+    sc = _scene("bilinear", min_upoly=0.02)
+    a = hostbuild.trace(sc, rays, world=False, dice_depth=14)
+    b = hostbuild.trace(sc, rays, world=False, dice_depth=0)
+    for k in ("t", "inst", "u", "v", "aux"):
+        assert np.array_equal(a[k], b[k]), k
