@@ -228,7 +228,7 @@ struct RenderLaunch {
     float bg[3];
     DevSpectrum spec;
 };
-constexpr int PATH_PLANES = 58;  // float planes of a path state
+constexpr int PATH_PLANES = 50;  // float planes of a path state
 // Path buffers of one chunk of `cap` paths: states (PATH_PLANES), two world
 // ray streams, hits, two active lists, counters (u32 x 4).
 struct RenderBuffers {
