@@ -103,15 +103,22 @@ void make_halton_tables(std::vector<HaltonDim>& t_dims, std::vector<uint16_t>& t
             }
             t_perm.push_back((uint16_t)result);
         }
-        uint64_t power = max_power / pow_base, div = 1;
+        // term n takes the index's digit n in base pow_base
+        uint64_t power = max_power / pow_base;
         uint32_t n = 0;
-        h.div[n] = 1; h.power[n] = (uint32_t)power; ++n;
+        h.power[n++] = (uint32_t)power;
         while (power / pow_base > 1) {
-            div *= pow_base; power /= pow_base;
-            h.div[n] = (uint32_t)div; h.power[n] = (uint32_t)power; ++n;
+            power /= pow_base;
+            h.power[n++] = (uint32_t)power;
         }
-        h.div[n] = (uint32_t)(div * pow_base); h.power[n] = 1; ++n;
+        h.power[n++] = 1;
         h.n_terms = n;
+        // with 2^l the power of two above pow_base (3 at least): magic =
+        // floor(2^32 (2^l - pow_base) / pow_base) + 1, shift = l - 1
+        uint32_t l = 0;
+        while ((1ull << l) < pow_base) ++l;
+        h.magic = (uint32_t)((((1ull << l) - pow_base) << 32) / pow_base + 1);
+        h.shift = l - 1;
         h.scale = 0x1.fffffep-1 / (double)max_power;
     }
 }

@@ -104,13 +104,14 @@ struct DevScene {
     uint32_t flags;           // PSY_SCENE_*
 };
 
-// Halton tables (dimension d >= 1): perm table offset, pow_base, terms.
+// Halton tables (dimension d >= 1): perm table offset, pow_base, digits, and
+// the reciprocal that divides by pow_base (halton_dim).
+constexpr uint32_t HALTON_TERMS = 7;  // most digits of any of the 256 dimensions (base 23)
 struct HaltonDim {
-    uint32_t perm_offset, pow_base, n_terms, pad;
-    uint32_t div[8];
-    uint32_t power[8];
+    uint32_t perm_offset, pow_base, n_terms, magic;
+    uint32_t power[HALTON_TERMS];
+    uint32_t shift;
     double scale;
-    double pad2;
 };
 
 struct DevHits { float* t; uint32_t* inst; float* u; float* v; float* aux; };
