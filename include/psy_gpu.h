@@ -233,7 +233,7 @@ typedef struct psy_scene_info {
 int psy_ctx_create(int device, psy_ctx** out);
 int psy_ctx_destroy(psy_ctx* ctx);
 /* Launch form of the trace's main pass (no counterpart in the reference,
- * whose tracer is a per-thread CPU loop).  PSY_TRACE_MODE_PLAIN (default):
+ * whose tracer is a per-thread CPU loop).  PSY_TRACE_MODE_PLAIN:
  * one thread per ray.  PSY_TRACE_MODE_PERSISTENT: one grid that fills the
  * GPU; each wave refills its finished lanes from a global ray counter once
  * refill_min (1..64) of its 64 lanes are idle; blocks_per_cu <= 0 takes the
@@ -241,8 +241,9 @@ int psy_ctx_destroy(psy_ctx* ctx);
  * of a wave advances only the lanes of its majority kind of work
  * (split-tree walk, or BVH node / leaf), so the wave issues one kind of
  * step at a time.  PSY_TRACE_MODE_PLAIN_COHERENT: one thread per ray, with
- * the same majority stepping (faster on instanced, moving and bicubic
- * scenes; the autotuner tries it).  Results are identical. */
+ * the same majority stepping (the autotuner tries it).  Unless one is set:
+ * plain coherent for world rays in a moving scene most of whose leaf
+ * instances are patches, else plain.  Results are identical. */
 #define PSY_TRACE_MODE_PLAIN 0
 #define PSY_TRACE_MODE_PERSISTENT 1
 #define PSY_TRACE_MODE_COHERENT 2
@@ -267,7 +268,8 @@ int psy_ctx_set_second_pass(psy_ctx* ctx, uint32_t wide_min, int32_t budget);
  * rays are still tracing (1..64), their traversal state goes to a
  * continuation buffer in the context's scratch and a follow-on launch
  * finishes them 64 to a wave; 0 turns it off.  Unless set, psy_trace_rays
- * continues below 24 and everything that traces world rays does not.
+ * of 2^21 rays or more continues below 24, and shorter streams and
+ * everything that traces world rays do not.  Plain coherent waves never do.
  * Results are identical.
  * psy_trace_rays_static never continues. */
 int psy_ctx_set_continuation(psy_ctx* ctx, int below);

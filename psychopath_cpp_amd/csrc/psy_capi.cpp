@@ -1206,6 +1206,9 @@ int psy_scene_create(psy_ctx* ctx, const psy_scene_desc* d, int dice_depth, psy_
     s.bvh1 = H.bvh1.empty() ? nullptr : s.bvh;
     s.n_bvh = (int32_t)H.bvh.size();
     s.root = H.root;
+    int64_t n_patch_insts = 0;
+    for (const DevInstance& in : H.insts) n_patch_insts += in.kind == K_BILINEAR || in.kind == K_BICUBIC ? 1 : 0;
+    s.mostly_patches = n_patch_insts > 0 && 2 * n_patch_insts >= (int64_t)H.insts.size() ? 1 : 0;
     s.inst = (const DevInstance*)sc->inst.p;
     s.obj = (const DevObject*)sc->obj.p;
     s.odata = (const float*)sc->odata.p;

@@ -91,6 +91,7 @@ struct DevScene {
                               // nodes' planes change with the ray's time
     int32_t n_bvh;
     int32_t root;             // child ref of the root (node 0, or a leaf)
+    int32_t mostly_patches = 0;  // half of the leaf instances or more are patches
     const DevInstance* inst;
     const DevObject* obj;
     const float* odata;
@@ -159,10 +160,17 @@ constexpr int32_t DEEP_BUDGET = 512;
 // How the main trace pass is launched: persistent (persist_blocks blocks,
 // lanes refilled when refill_min of a wave's 64 are idle) or one thread per
 // ray.
+// Calls of fewer object rays continue none by default: the follow-on launch
+// is a latency of its own.  Below, continuations have cost 8 to 45 % (121x104x2
+// camera rays 110 us for 79, 2^19 bounce rays 608 for 551, 2^20 940 for 929);
+// from here a stream of bounce rays takes 1 to 5 % less (2^21 1.84 ms for
+// 1.87, 2^23 6.63 for 6.97).
+constexpr int64_t CONT_MIN_RAYS = (int64_t)1 << 21;
 struct TraceTuning {
     bool persistent;
     bool coherent = false;  // persistent: step one kind of work per wave step
     bool plain_coherent = false;  // one thread per ray, stepping one kind of work per wave step
+    bool auto_form = false;       // one thread per ray, stepped so where that pays (launch_trace_w)
     int persist_blocks;    // persistent grid with the 16-entry stack
     int persist_blocks32;  // and with the 32-entry stack
     int refill_min;
@@ -179,6 +187,7 @@ struct TraceTuning {
     uint32_t* cont = nullptr;
     int64_t cont_words = 0;
     int cont_below = 0;
+    int64_t cont_min = 0;  // calls of fewer rays continue none
     // hipEvent_t handles recorded around the passes when the context times
     // them: before the main pass, after it, after the second pass.
     void* ev[3] = {nullptr, nullptr, nullptr};

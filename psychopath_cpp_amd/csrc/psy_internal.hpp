@@ -100,16 +100,18 @@ struct psy_ctx {
     int occupancy32[2] = {0, 0};  // 32-entry stack
     int trace_stack = 16;         // main-pass LDS stack entries
     // main pass: continue a wave's rays once fewer lanes trace (0: never).
-    // By default (CONT_DEFAULT) DEFAULT_CONT_BELOW for object rays, never for
-    // world rays: saving and restoring a ray costs more the more it carries
-    // and the less it still has to do.  Without continuations the object
-    // stream of 2^22 rays takes 1.91 ms for 1.86, but a million shadow rays
-    // (world form) 0.11 ms for 0.26, and the renders, all in world form, 1 to
-    // 20 % less (spheres 256x256x16 1.62 ms for 2.01, heightfield
-    // 1024x1024x16 51.9 for 52.9).
+    // By default (CONT_DEFAULT) DEFAULT_CONT_BELOW for CONT_MIN_RAYS object
+    // rays and more, never for world rays: saving and restoring a ray costs
+    // more the more it carries and the less it still has to do (a million
+    // shadow rays, in world form, 0.11 ms without for 0.26, and the renders,
+    // all in world form, 1 to 20 % less: spheres 256x256x16 1.62 ms for 2.01,
+    // heightfield 1024x1024x16 51.9 for 52.9).
     static constexpr int CONT_DEFAULT = -1, DEFAULT_CONT_BELOW = 24;
     int cont_below = CONT_DEFAULT;
-    int mode = PSY_TRACE_MODE_PLAIN;
+    // main-pass form: MODE_DEFAULT (plain, or plain coherent where that pays:
+    // launch_trace_w) until psy_ctx_set_trace_mode picks one
+    static constexpr int MODE_DEFAULT = -1;
+    int mode = MODE_DEFAULT;
     int refill_min = 16;
     int blocks_per_cu = 0;  // <= 0: from occupancy
     // pass timing: event triples of the trace calls since the last query
@@ -120,6 +122,7 @@ struct psy_ctx {
         t.persistent = mode == PSY_TRACE_MODE_PERSISTENT || mode == PSY_TRACE_MODE_COHERENT;
         t.coherent = mode == PSY_TRACE_MODE_COHERENT;
         t.plain_coherent = mode == PSY_TRACE_MODE_PLAIN_COHERENT;
+        t.auto_form = mode == MODE_DEFAULT && (!world || cont_below == CONT_DEFAULT);
         t.persist_blocks = n_cu * (blocks_per_cu > 0 ? blocks_per_cu : occupancy[world ? 1 : 0]);
         t.persist_blocks32 = n_cu * (blocks_per_cu > 0 ? blocks_per_cu : occupancy32[world ? 1 : 0]);
         t.refill_min = refill_min;
@@ -130,6 +133,7 @@ struct psy_ctx {
             t.cont = (uint32_t*)queue.p + 6 * queue_cap;
             t.cont_words = psy::cont_area_words(queue_cap);
             t.cont_below = cont_below != CONT_DEFAULT ? cont_below : (world ? 0 : DEFAULT_CONT_BELOW);
+            t.cont_min = cont_below != CONT_DEFAULT ? 0 : psy::CONT_MIN_RAYS;
         }
         if (timing && timed) {
             for (int k = 0; k < 3; ++k) {
