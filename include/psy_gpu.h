@@ -278,7 +278,7 @@ int psy_ctx_set_continuation(psy_ctx* ctx, int below);
  * one; the default 2^21 paths.  Results do not depend on it. */
 int psy_ctx_set_render_chunk(psy_ctx* ctx, int64_t paths);
 /* Chunks of PSY_RENDER_WAVEFRONT in flight at once (no counterpart in the
- * reference): 1..4, default 2.  With k > 1, a render of more than one chunk
+ * reference): 1..4, default 4.  With k > 1, a render of more than one chunk
  * runs up to k chunks at once, each beyond the first on a stream of the
  * context's own with scratch of its own (a set of path, ray and trace
  * buffers per chunk: k times the render scratch), and the host queues each
@@ -286,7 +286,8 @@ int psy_ctx_set_render_chunk(psy_ctx* ctx, int64_t paths);
  * chunk's short late bounces run beside the others' work.  The caller's
  * stream waits for all of them at the end.  While such a render runs, the
  * calling thread polls the chunks' events (one host core stays busy).
- * Same samples as with 1. */
+ * Where memory is short a render takes fewer, down to 2.  Same samples as
+ * with 1. */
 int psy_ctx_set_render_streams(psy_ctx* ctx, int streams);
 /* Register budget of PSY_RENDER_WAVEFRONT's shading kernel for the steps
  * that take a hit and sample a light (no counterpart in the reference):

@@ -460,9 +460,16 @@ int alloc_render(psy_ctx* ctx, bool own_samples, int64_t extra_floats, RenderSet
             if (!e) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     }
     for (int k = 0; k + 1 < U.slots; ++k) {
-        if (int rc = ctx->slot_scratch[k].reserve((size_t)f_slot * sizeof(float))) return rc;
-        if (int rc = ensure_trace_scratch(ctx->slot_queue[k], ctx->slot_counters[k], ctx->slot_queue_cap[k], cap))
-            return rc;
+        int rc = ctx->slot_scratch[k].reserve((size_t)f_slot * sizeof(float));
+        if (!rc) rc = ensure_trace_scratch(ctx->slot_queue[k], ctx->slot_counters[k], ctx->slot_queue_cap[k], cap);
+        if (rc && k >= 1) {
+            // no memory for a third or fourth chunk: go on with those there are
+            (void)hipGetLastError();
+            ctx->slot_scratch[k].release();
+            U.slots = k + 1;
+            break;
+        }
+        if (rc) return rc;
         if (!ctx->slot_stream[k]) HIP_OK(hipStreamCreateWithFlags(&ctx->slot_stream[k], hipStreamNonBlocking));
         carve_slot((float*)ctx->slot_scratch[k].p, cap, own_samples, U.Bx[k], &U.samples_x[k]);
     }
@@ -1040,7 +1047,13 @@ int psy_adjoint(psy_ctx* ctx, const psy_scene* s, const psy_render_params* prm, 
     const int64_t f_q = (int64_t)ADJ_STATE_PLANES * U.cap;
     const int64_t f_grad = (n_params + 63) / 64 * 64;
     const int64_t f_part = J.lds ? (int64_t)J.rows * n_params : 0;
-    if (int rc = alloc_render(ctx, true, U.slots * (f_q + f_part) + f_grad, U)) return rc;
+    int rc_alloc = alloc_render(ctx, true, U.slots * (f_q + f_part) + f_grad, U);
+    if (rc_alloc && U.slots > 2) {  // with less memory, two chunks
+        (void)hipGetLastError();
+        U.slots = 2;
+        rc_alloc = alloc_render(ctx, true, U.slots * (f_q + f_part) + f_grad, U);
+    }
+    if (rc_alloc) return rc_alloc;
     J.q = U.extra;
     J.grad = J.q + U.slots * f_q;
     J.partials = J.grad + f_grad;
