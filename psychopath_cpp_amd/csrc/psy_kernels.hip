@@ -256,8 +256,9 @@ __global__ void k_zero_n(uint32_t* p, int n) {
     if (i < n) p[i] = 0u;
 }
 
-__global__ void k_zero_counters(uint32_t* p) {
+__global__ void k_zero_counters(uint32_t* p, uint32_t* also) {
     if (threadIdx.x < 8 && blockIdx.x == 0) p[threadIdx.x] = 0u;
+    if (also && threadIdx.x == 8 && blockIdx.x == 0) *also = 0u;
 }
 
 // Intersection records of the hits of world rays (PSY_ISECT_PLANES planes
@@ -830,7 +831,7 @@ static int launch_trace_w(const DevScene& s, int stack_need, const float* rays, 
     // deep-node pool (n entries of 3 words)
     uint32_t* heads = queue + 2 * n;
     const DeepPool pool{queue + 3 * n, counters + 4, (uint32_t)std::min<int64_t>(n, (int64_t)UINT32_MAX - 2)};
-    hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, counters);
+    hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, counters, tune.zero_also);
     if (tune.ev[0]) (void)hipEventRecord((hipEvent_t)tune.ev[0], st);
     const ContBuf no_cont{nullptr, 0u, 0, counters + 5};
     const int64_t plain_blocks = grid_for(n, TRACE_BLOCK);

@@ -552,12 +552,12 @@ int run_wavefront(psy_ctx* ctx, const psy_scene* s, const psy_render_params* prm
     auto step = [&](ChunkSlot& c) -> int {
         traced += c.n_active;
         TraceTuning t = ctx->tuning(true);
+        t.zero_also = c.B.count + (c.cur ^ 1);
         t.cont = c.queue + 6 * c.queue_cap;
         t.cont_words = cont_area_words(c.queue_cap);
         int rc = launch_trace(s->dev, true, false, s->stack_need, c.B.rays[c.cur], c.n_active, c.B.cap, c.B.hits,
                               c.queue, c.counters, t, c.st);
         if (rc) return fail(rc, "psy_render: trace launch failed");
-        if ((rc = launch_zero_u32(c.B.count + (c.cur ^ 1), 1, c.st))) return fail(rc, "psy_render: launch failed");
         float* samp = sample_xyz ? sample_xyz : c.samples;
         const int64_t sbase = sample_xyz ? 0 : c.first;
         rc = adj ? launch_render_adjoint(R, c.first, c.B, adj[&c - S], c.cur, c.n_active, c.step, c.st)
@@ -703,9 +703,9 @@ int capture_steps(psy_ctx* ctx, const psy_scene* s, const RenderLaunch& R, const
     for (int it = 0; it < iters && !rc; ++it) {
         const int cur = it & 1;
         tune.n_dev = &S->count[cur];
+        tune.zero_also = &S->count[cur ^ 1];
         rc = launch_trace(s->dev, true, false, s->stack_need, B.rays[cur], U.cap, U.cap, B.hits,
                           (uint32_t*)ctx->queue.p, (uint32_t*)ctx->counters.p, tune, cs);
-        if (!rc) rc = launch_zero_u32(&S->count[cur ^ 1], 1, cs);
         if (!rc) rc = launch_stream_shade(R, B, cur, S, wait, blocks, samp, sbase, cs);
         if (!rc && cur) rc = launch_zero_u32(&S->n_wait, 1, cs);  // the odd step refilled every parked slot
     }

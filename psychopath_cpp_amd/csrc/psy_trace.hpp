@@ -60,7 +60,7 @@ PSY_DEV void halton_digit(PSY_CONST_AS const HaltonDim* h, uint32_t t, const uin
 // One dimension for one index.  A chain of dependent loads and divisions is
 // what bounded the steps that draw few other values: with the digits chained
 // and the constants from the scalar cache the heightfield render takes 49.4
-// ms for 50.3, the nested spheres 1.42 for 1.47, a 256x256 preview 583 us
+// ms for 50.3, the nested spheres 1.42 for 1.47, a 96x64 preview 583 us
 // for 606.  Every dimension has 3 to 7 digits; the first
 // four are straight-line (a fourth that a dimension does not have weighs 0),
 // so that their table reads are in flight together.
