@@ -620,70 +620,10 @@ struct Builder2 {
     }
 };
 
-// ---- outward-rounded f16 planes ---------------------------------------------
-constexpr uint16_t F16_PINF = 0x7c00, F16_NINF = 0xfc00;
-// The next f16 value below h.
-uint16_t f16_below(uint16_t h) {
-    if (h == F16_NINF) return h;
-    if (h & 0x8000u) return (uint16_t)(h + 1);
-    return h == 0 ? (uint16_t)0x8001u : (uint16_t)(h - 1);
-}
-// The largest f16 value not above x (NaN: -inf).
-uint16_t f16_floor(double x) {
-    if (!(x >= -65504.0)) return F16_NINF;
-    if (x >= 65504.0) return x == (double)INFINITY ? F16_PINF : (uint16_t)0x7bff;
-    int e = 0;
-    if (x != 0.0) (void)std::frexp(std::fabs(x), &e);  // |x| = m 2^e, m in [0.5, 1)
-    const int u = std::max(e - 11, -24);               // the exponent of a unit in the last place
-    double q = std::floor(std::ldexp(x, -u));          // |q| <= 2048
-    if (q == 0.0) return 0;
-    const bool neg = q < 0.0;
-    q = std::fabs(q);
-    int k = u;
-    if (q == 2048.0) { q = 1024.0; ++k; }
-    const uint16_t m = (uint16_t)q;
-    const uint16_t bits = m < 1024 ? m : (uint16_t)(((k + 25) << 10) | (m - 1024));
-    return (uint16_t)(neg ? bits | 0x8000u : bits);
-}
-uint16_t f16_lo(double x) { return f16_below(f16_floor(x)); }
-uint16_t f16_hi(double x) { return (uint16_t)(f16_lo(-x) ^ 0x8000u); }
-
-// Packs the boxes of up to 4 children at time 0 (b) and time 1 (e) into a node.
-void pack_node(const Box* const* b, const Box* const* e, int n, BvhNode& o) {
-    double far = 0.0;
-    for (int a = 0; a < 3; ++a) {
-        float lo = INFINITY, hi = -INFINITY;
-        for (int k = 0; k < n; ++k) { lo = std::min(lo, b[k]->lo[a]); hi = std::max(hi, b[k]->hi[a]); }
-        const float mid = (float)(0.5 * ((double)lo + (double)hi));
-        o.org[a] = std::isfinite(mid) ? mid : 0.0f;
-        for (int k = 0; k < n; ++k)
-            for (const double x : {(double)b[k]->lo[a] - o.org[a], (double)b[k]->hi[a] - o.org[a],
-                                   (double)e[k]->lo[a] - b[k]->lo[a], (double)e[k]->hi[a] - b[k]->hi[a]})
-                if (std::isfinite(x)) far = std::max(far, std::fabs(x));
-    }
-    // offsets of at most 2^14 units, with f16's full precision down to 2^-28
-    // of the largest
-    int ex = 0;
-    if (far > 0.0) { (void)std::frexp(far, &ex); ex = std::max(ex - 14, -100); }
-    o.scale = (float)std::ldexp(1.0, ex);
-    for (int a = 0; a < 3; ++a)
-        for (int k = 0; k < 4; ++k) {
-            if (k < n) {
-                o.plane[a][k] = f16_lo(std::ldexp((double)b[k]->lo[a] - o.org[a], -ex));
-                o.plane[a][4 + k] = f16_hi(std::ldexp((double)b[k]->hi[a] - o.org[a], -ex));
-                o.delta[a][k] = f16_lo(std::ldexp((double)e[k]->lo[a] - b[k]->lo[a], -ex));
-                o.delta[a][4 + k] = f16_hi(std::ldexp((double)e[k]->hi[a] - b[k]->hi[a], -ex));
-            } else {  // never hit
-                o.plane[a][k] = F16_PINF;
-                o.plane[a][4 + k] = F16_NINF;
-                o.delta[a][k] = o.delta[a][4 + k] = 0;
-            }
-        }
-}
-
 struct Collapser {
     const std::vector<B2>* n2;
-    std::vector<BvhNode> out;
+    std::vector<BvhNode> out;   // child boxes at time 0
+    std::vector<BvhNode> out1;  // the same nodes: child box change from time 0 to 1
     int max_need = 0;
     // which binary child a 4-wide node opens up next: the largest surface
     // area (the SAH's choice), or with by_count the most leaves (halves the
@@ -712,6 +652,7 @@ struct Collapser {
         }
         const int me = (int)out.size();
         out.emplace_back();
+        out1.emplace_back();
         int32_t refs[4];
         int sub_need = 0;
         for (int k = 0; k < 4; ++k) {
@@ -723,14 +664,29 @@ struct Collapser {
                 refs[k] = CHILD_EMPTY;
             }
         }
-        const Box *b[4], *e[4];
-        const int kc = (int)kids.size();
-        for (int k = 0; k < kc; ++k) {
-            b[k] = &(*n2)[kids[k]].box0;
-            e[k] = &(*n2)[kids[k]].box1;
+        // out: child boxes at time 0; out1: their change up to time 1
+        // (0 for empty slots, whose +inf / -inf then stay put)
+        BvhNode& o = out[me];
+        BvhNode& o1 = out1[me];
+        for (int k = 0; k < 4; ++k) {
+            o.child[k] = o1.child[k] = refs[k];
+            if (k < (int)kids.size()) {
+                const Box& b = (*n2)[kids[k]].box0;
+                const Box& e = (*n2)[kids[k]].box1;
+                o.lo_x[k] = b.lo[0]; o.hi_x[k] = b.hi[0];
+                o.lo_y[k] = b.lo[1]; o.hi_y[k] = b.hi[1];
+                o.lo_z[k] = b.lo[2]; o.hi_z[k] = b.hi[2];
+                o1.lo_x[k] = e.lo[0] - b.lo[0]; o1.hi_x[k] = e.hi[0] - b.hi[0];
+                o1.lo_y[k] = e.lo[1] - b.lo[1]; o1.hi_y[k] = e.hi[1] - b.hi[1];
+                o1.lo_z[k] = e.lo[2] - b.lo[2]; o1.hi_z[k] = e.hi[2] - b.hi[2];
+            } else {
+                o.lo_x[k] = o.lo_y[k] = o.lo_z[k] = INFINITY;
+                o.hi_x[k] = o.hi_y[k] = o.hi_z[k] = -INFINITY;
+                o1.lo_x[k] = o1.lo_y[k] = o1.lo_z[k] = 0.0f;
+                o1.hi_x[k] = o1.hi_y[k] = o1.hi_z[k] = 0.0f;
+            }
         }
-        pack_node(b, e, kc, out[me]);
-        for (int k = 0; k < 4; ++k) out[me].child[k] = refs[k];
+        const int kc = (int)kids.size();
         *need = std::max(kc, kc - 1 + sub_need);
         return me;
     }
@@ -1073,7 +1029,7 @@ int prepare_scene(const psy_scene_desc* d, int dice_depth, HostScene& H) {
             return fail(PSY_ERR_UNSUPPORTED, "psy_scene_create: the instance BVH needs a traversal stack of " +
                                                  std::to_string(stack_need) + " entries; at most 64 are supported");
         bvh.swap(cl.out);
-        if (moving) H.bvh1.resize(1);
+        if (moving) H.bvh1.swap(cl.out1);
     }
     H.root = root;
     H.stack_need = stack_need;
@@ -1176,6 +1132,7 @@ int psy_scene_create(psy_ctx* ctx, const psy_scene_desc* d, int dice_depth, psy_
     // ---- upload ------------------------------------------------------------
     int rc;
     if ((rc = sc->bvh.upload(H.bvh))) return rc;
+    if (!H.bvh1.empty() && (rc = sc->bvh1.upload(H.bvh1))) return rc;
     if ((rc = sc->inst.upload(H.insts))) return rc;
     if ((rc = sc->obj.upload(H.objs))) return rc;
     if ((rc = sc->odata.upload(H.odata))) return rc;
@@ -1203,7 +1160,7 @@ int psy_scene_create(psy_ctx* ctx, const psy_scene_desc* d, int dice_depth, psy_
 
     DevScene& s = sc->dev;
     s.bvh = (const BvhNode*)sc->bvh.p;
-    s.bvh1 = H.bvh1.empty() ? nullptr : s.bvh;
+    s.bvh1 = H.bvh1.empty() ? nullptr : (const BvhNode*)sc->bvh1.p;
     s.n_bvh = (int32_t)H.bvh.size();
     s.root = H.root;
     int64_t n_patch_insts = 0;
@@ -1229,7 +1186,7 @@ int psy_scene_create(psy_ctx* ctx, const psy_scene_desc* d, int dice_depth, psy_
     info.dice_depth = levels;
     info.bvh_stack_need = H.stack_need;
     info.dice_cache_bytes = (int64_t)dice_bytes;
-    info.device_bytes = (int64_t)(sc->bvh.bytes + sc->inst.bytes + sc->obj.bytes + sc->odata.bytes + sc->xf.bytes +
+    info.device_bytes = (int64_t)(sc->bvh.bytes + sc->bvh1.bytes + sc->inst.bytes + sc->obj.bytes + sc->odata.bytes + sc->xf.bytes +
                                   sc->shaders.bytes + dice_bytes);
     *out = sc.release();
     return PSY_OK;

@@ -2,11 +2,10 @@
 // interface between the host library and the HIP kernels.
 //
 // Layout (all arrays in device memory, read-only after psy_scene_create):
-//   bvh    : BVH4 over flattened leaf instances, 128-byte nodes (one L2
-//            line each); child boxes stored per axis as 4-wide lanes (the
-//            reference BBox4 layout, basics/bbox.hpp:461-476) of f16
-//            offsets, 16 bytes of child refs, and for moving scenes the
-//            boxes' change over the shutter.
+//   bvh    : BVH4 over flattened leaf instances, 128-byte nodes; child
+//            boxes stored per axis as 4-wide lanes (the reference BBox4
+//            layout, basics/bbox.hpp:461-476), 16 bytes of child refs,
+//            16 bytes of padding (one node = one 128-byte L2 line).
 //   inst   : 32-byte leaf-instance records (object, merged transforms,
 //            effective shader, and for patches the dice-cache slot, so a
 //            traversal reaching a patch leaf reads one record) -- the
@@ -31,22 +30,10 @@ enum : int32_t {
 constexpr int32_t CHILD_EMPTY = INT32_MIN;  // unused BVH4 lane
 // child ref: >= 0 inner node index; < 0 and != CHILD_EMPTY: leaf ~ref
 
-// A node's child planes are f16 offsets from the node's own origin, in units
-// of its power-of-two scale, rounded outwards by one unit in the last place
-// at least (psy_capi.cpp), so the stored boxes hold the exact ones with room
-// for the rounding of the traversal's float arithmetic.  A visit to a static
-// node reads 80 bytes, 5 16-byte loads, where float planes took 7: what
-// bounds the traversal next to instruction issue is the width of the data
-// path back from the L1 (a wave's 16-byte load takes 16 clocks of it however
-// few lanes are active, 27 with a quarter of them, 54 with all).  The changes
-// of a moving scene's planes lie in the same cache line, where a second
-// array of nodes took another.
 struct alignas(16) BvhNode {
-    float org[3];
-    float scale;
-    uint16_t plane[3][8];  // x, y, z: the children's low planes, then their high planes
+    float lo_x[4], hi_x[4], lo_y[4], hi_y[4], lo_z[4], hi_z[4];
     int32_t child[4];
-    uint16_t delta[3][8];  // change of each plane from time 0 to time 1, rounded the same way
+    int32_t pad[4];  // keeps nodes 128-byte aligned
 };
 static_assert(sizeof(BvhNode) == 128, "BVH node must be 128 bytes");
 
@@ -87,8 +74,9 @@ struct DevCamera {
 // Everything a kernel needs to trace against a scene (passed by value).
 struct DevScene {
     const BvhNode* bvh;
-    const BvhNode* bvh1;      // not null for a scene with moving leaves: its
-                              // nodes' planes change with the ray's time
+    const BvhNode* bvh1;      // moving scenes: each node's child box change
+                              // from time 0 (bvh) to time 1, which a ray
+                              // scales by its time; null for static scenes
     int32_t n_bvh;
     int32_t root;             // child ref of the root (node 0, or a leaf)
     int32_t mostly_patches = 0;  // half of the leaf instances or more are patches

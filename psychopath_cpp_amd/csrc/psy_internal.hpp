@@ -202,7 +202,7 @@ struct psy_scene {
     int device = 0;  // the context's device (the scene may outlive its context)
     psy::DevScene dev{};
     psy::DevCamera cam{};
-    psy::DBuf bvh, inst, obj, odata, xf, dice, shaders;
+    psy::DBuf bvh, bvh1, inst, obj, odata, xf, dice, shaders;
     // differentiable parameters: shader albedos (host copy of the table),
     // emission scales of the light objects
     std::vector<psy::DevShader> host_shaders;
@@ -233,7 +233,7 @@ namespace psy {
 // built on the device) and the light trees.
 struct HostScene {
     std::vector<BvhNode> bvh;
-    std::vector<BvhNode> bvh1;  // not empty when some leaf moves (a marker: the nodes hold the changes)
+    std::vector<BvhNode> bvh1;  // child box change to time 1 when some leaf moves
     int32_t root = CHILD_EMPTY;
     int stack_need = 1;
     std::vector<DevInstance> insts;

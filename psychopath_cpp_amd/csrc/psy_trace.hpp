@@ -689,106 +689,35 @@ struct TRay {
     bool occl;
 };
 
-// ---- f16 planes of a BVH4 node -----------------------------------------------
-// Child c's value in a packed axis (c 0..3 of four f16 in two words).  On the
-// device a f16 operand of a fused multiply-add needs no conversion.
-#if defined(__HIP_DEVICE_COMPILE__)
-typedef _Float16 HalfPair __attribute__((ext_vector_type(2)));
-#endif
-PSY_DEV float f16_at(uint32_t w, int hi) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    HalfPair h;
-    __builtin_memcpy(&h, &w, 4);
-    return hi ? (float)h.y : (float)h.x;
-#else
-    const uint32_t h = hi ? w >> 16 : w & 0xffffu;
-    const uint32_t e = (h >> 10) & 31u, m = h & 1023u;
-    const float v = e == 31 ? (m ? __builtin_nanf("") : INFINITY)
-                            : ldexpf((float)(e ? m | 1024u : m), (int)(e ? e : 1u) - 25);
-    return (h & 0x8000u) ? -v : v;
-#endif
-}
-
-// The near and far planes of a node's children along one axis, two children
-// a word, for a ray whose direction is negative there or not.
-struct AxisPlanes { uint32_t n01, n23, f01, f23; };
-PSY_DEV AxisPlanes axis_planes(const uint16_t* p, bool neg) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    return AxisPlanes{neg ? v.z : v.x, neg ? v.w : v.y, neg ? v.x : v.z, neg ? v.y : v.w};
-}
-
-// Slab distances of the four children along an axis: (origin - o) / d +
-// offset * scale / d, with one rounding of that sum (c and sd are its ray
-// terms).  Moving scenes add the planes' change up to the ray's time.
-struct AxisT { float n[4], f[4]; };
-PSY_DEV AxisT axis_t(const AxisPlanes& p, float sd, float c) {
-    return AxisT{{__builtin_fmaf(f16_at(p.n01, 0), sd, c), __builtin_fmaf(f16_at(p.n01, 1), sd, c),
-                  __builtin_fmaf(f16_at(p.n23, 0), sd, c), __builtin_fmaf(f16_at(p.n23, 1), sd, c)},
-                 {__builtin_fmaf(f16_at(p.f01, 0), sd, c), __builtin_fmaf(f16_at(p.f01, 1), sd, c),
-                  __builtin_fmaf(f16_at(p.f23, 0), sd, c), __builtin_fmaf(f16_at(p.f23, 1), sd, c)}};
-}
-PSY_DEV float moved(uint32_t p, uint32_t d, int hi, float time) {
-    return __builtin_fmaf(f16_at(d, hi), time, f16_at(p, hi));
-}
-PSY_DEV AxisT axis_t_moving(const AxisPlanes& p, const AxisPlanes& d, float time, float sd, float c) {
-    return AxisT{{__builtin_fmaf(moved(p.n01, d.n01, 0, time), sd, c), __builtin_fmaf(moved(p.n01, d.n01, 1, time), sd, c),
-                  __builtin_fmaf(moved(p.n23, d.n23, 0, time), sd, c), __builtin_fmaf(moved(p.n23, d.n23, 1, time), sd, c)},
-                 {__builtin_fmaf(moved(p.f01, d.f01, 0, time), sd, c), __builtin_fmaf(moved(p.f01, d.f01, 1, time), sd, c),
-                  __builtin_fmaf(moved(p.f23, d.f23, 0, time), sd, c), __builtin_fmaf(moved(p.f23, d.f23, 1, time), sd, c)}};
-}
-// A box found hit by its exact planes is found hit by the packed ones: where
-// a plane is far from the node's origin (against the ray's distance from it)
-// the outward rounding covers the difference in float rounding, and where it
-// is near, the two distances agree to 2^-22, which these factors cover.
-#define PSY_NODE_NEAR 0.9999995f
-#define PSY_NODE_FAR 1.000001f
-// Whether a ray's distances to every node of the scene stay well inside the
-// float range (no infinity minus infinity); other rays take the second pass.
-PSY_DEV bool nodes_in_range(const DevScene& s, V3 o, V3 dinv) {
-    if (s.root < 0) return true;  // a leaf or nothing: no node to visit
-    const BvhNode& r = s.bvh[s.root];
-    const float e = r.scale * 262144.0f;  // 16 times the offsets' limit
-    return (fabsf(r.org[0]) + fabsf(o.x) + e) * fabsf(dinv.x) < 1e37f &&
-           (fabsf(r.org[1]) + fabsf(o.y) + e) * fabsf(dinv.y) < 1e37f &&
-           (fabsf(r.org[2]) + fabsf(o.z) + e) * fabsf(dinv.z) < 1e37f;
-}
-
-// A node's child boxes as floats, for the passes that follow the reference's
-// slab test through infinities and NaN: the planes as near / far per axis for
-// the ray's direction signs (ds*: that component of the inverse direction is
-// negative).  origin + offset is rounded once, which keeps it on the outer
-// side of the exact plane, a float itself.
-PSY_DEV float4 plane_floats(uint32_t p01, uint32_t p23, float scale, float org) {
-    return make_float4(__builtin_fmaf(f16_at(p01, 0), scale, org), __builtin_fmaf(f16_at(p01, 1), scale, org),
-                       __builtin_fmaf(f16_at(p23, 0), scale, org), __builtin_fmaf(f16_at(p23, 1), scale, org));
-}
-PSY_DEV float4 plane_floats_moving(uint32_t p01, uint32_t p23, uint32_t d01, uint32_t d23, float time, float scale,
-                                   float org) {
-    return make_float4(__builtin_fmaf(moved(p01, d01, 0, time), scale, org),
-                       __builtin_fmaf(moved(p01, d01, 1, time), scale, org),
-                       __builtin_fmaf(moved(p23, d23, 0, time), scale, org),
-                       __builtin_fmaf(moved(p23, d23, 1, time), scale, org));
-}
+// A BVH4 node's child boxes at the ray's time: the stored boxes for a
+// static scene; for a moving one, the time-0 boxes plus the ray's time
+// (clamped to the shutter, as the transforms are) times their change up to
+// time 1.  Each endpoint box is the union of its subtree's, padded on the
+// host so the interpolation holds every leaf at every time (and the pad
+// covers the rounding of the two operations here).
+//
+// The planes come back as near / far per axis for the ray's direction
+// signs (ds*: that component of the inverse direction is negative, so the
+// max plane is met first): each lane loads them from its own offsets
+// instead of loading min and max and selecting per child.
 PSY_DEV void node_boxes(const DevScene& s, int32_t ref, float time, bool ds0, bool ds1, bool ds2, float4& nx,
                         float4& fx, float4& ny, float4& fy, float4& nz, float4& fz) {
-    const BvhNode& nd = s.bvh[ref];
-    const AxisPlanes x = axis_planes(nd.plane[0], ds0), y = axis_planes(nd.plane[1], ds1),
-                     z = axis_planes(nd.plane[2], ds2);
-    const float sc = nd.scale;
+    // 32-bit byte offsets from the (wave-uniform) array base
+    const uint32_t o = (uint32_t)ref * (uint32_t)sizeof(BvhNode);
+    const uint32_t ix = ds0 ? 16u : 0u, iy = ds1 ? 48u : 32u, iz = ds2 ? 80u : 64u;
+    const char* b = reinterpret_cast<const char*>(s.bvh);
+#define PSY_AT(B, OFF) (*reinterpret_cast<const float4*>((B) + (OFF)))
+    nx = PSY_AT(b, o + ix); fx = PSY_AT(b, o + (ix ^ 16u)); ny = PSY_AT(b, o + iy); fy = PSY_AT(b, o + (iy ^ 16u));
+    nz = PSY_AT(b, o + iz); fz = PSY_AT(b, o + (iz ^ 16u));
     if (s.bvh1) {
-        const AxisPlanes dx = axis_planes(nd.delta[0], ds0), dy = axis_planes(nd.delta[1], ds1),
-                         dz = axis_planes(nd.delta[2], ds2);
+        const char* b1 = reinterpret_cast<const char*>(s.bvh1);
         const float t = fminf(fmaxf(time, 0.0f), 1.0f);
-        nx = plane_floats_moving(x.n01, x.n23, dx.n01, dx.n23, t, sc, nd.org[0]);
-        fx = plane_floats_moving(x.f01, x.f23, dx.f01, dx.f23, t, sc, nd.org[0]);
-        ny = plane_floats_moving(y.n01, y.n23, dy.n01, dy.n23, t, sc, nd.org[1]);
-        fy = plane_floats_moving(y.f01, y.f23, dy.f01, dy.f23, t, sc, nd.org[1]);
-        nz = plane_floats_moving(z.n01, z.n23, dz.n01, dz.n23, t, sc, nd.org[2]);
-        fz = plane_floats_moving(z.f01, z.f23, dz.f01, dz.f23, t, sc, nd.org[2]);
-    } else {
-        nx = plane_floats(x.n01, x.n23, sc, nd.org[0]); fx = plane_floats(x.f01, x.f23, sc, nd.org[0]);
-        ny = plane_floats(y.n01, y.n23, sc, nd.org[1]); fy = plane_floats(y.f01, y.f23, sc, nd.org[1]);
-        nz = plane_floats(z.n01, z.n23, sc, nd.org[2]); fz = plane_floats(z.f01, z.f23, sc, nd.org[2]);
+        const float4 a0 = PSY_AT(b1, o + ix), a1 = PSY_AT(b1, o + (ix ^ 16u)), a2 = PSY_AT(b1, o + iy),
+                     a3 = PSY_AT(b1, o + (iy ^ 16u)), a4 = PSY_AT(b1, o + iz), a5 = PSY_AT(b1, o + (iz ^ 16u));
+#undef PSY_AT
+#define PSY_MIX(V, W) V = make_float4(V.x + W.x * t, V.y + W.y * t, V.z + W.z * t, V.w + W.w * t)
+        PSY_MIX(nx, a0); PSY_MIX(fx, a1); PSY_MIX(ny, a2); PSY_MIX(fy, a3); PSY_MIX(nz, a4); PSY_MIX(fz, a5);
+#undef PSY_MIX
     }
 }
 
@@ -973,7 +902,7 @@ PSY_DEV bool trace_one(const DevScene& s, const float* __restrict__ rays, int64_
         if (ref >= 0) {
             float4 nx, fx, ny, fy, nz, fz;
             node_boxes(s, ref, r.time, ds0, ds1, ds2, nx, fx, ny, fy, nz, fz);
-            const int4 ch = *reinterpret_cast<const int4*>(s.bvh[ref].child);
+            const int4 ch = reinterpret_cast<const int4*>(s.bvh + ref)[6];
             // BBox4::intersect_ray lanes (basics/bbox.hpp:566-595); keys are
             // the near distances of hit children, +inf otherwise
 #define PSY_LANE(L, KEY)                                                                             \
@@ -1261,9 +1190,9 @@ PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i) {
     L.state = 0;
     L.deep_head = DEEP_NONE;
     L.wframe = -1;  // read by world rays only
-    // the main pass's box tests assume a finite inverse direction and
-    // distances that stay finite; the second pass follows the reference's NaN behaviour exactly
-    bool plain = finite3(L.r.dinv) && nodes_in_range(s, L.r.o, L.r.dinv);
+    // the main pass's box tests assume a finite inverse direction; the
+    // second pass follows the reference's NaN behaviour exactly
+    bool plain = finite3(L.r.dinv);
     if (!WORLD) plain = make_foot(L.r.w, L.foot) && plain;
     if (!plain) {
         L.state = LANE_RETRACE;
@@ -1397,41 +1326,29 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
     if (ref >= 0) {
         const TRay& r = L.r;
         const bool ds0 = r.dinv.x < 0.0f, ds1 = r.dinv.y < 0.0f, ds2 = r.dinv.z < 0.0f;
-        // 32-bit byte offset from the (wave-uniform) array base
-        const BvhNode& nd = *reinterpret_cast<const BvhNode*>(reinterpret_cast<const char*>(s.bvh) +
-                                                              (uint32_t)ref * (uint32_t)sizeof(BvhNode));
-        const float4 os = *reinterpret_cast<const float4*>(nd.org);
-        const AxisPlanes px = axis_planes(nd.plane[0], ds0), py = axis_planes(nd.plane[1], ds1),
-                         pz = axis_planes(nd.plane[2], ds2);
-        const int4 ch = *reinterpret_cast<const int4*>(nd.child);
-        const float cx = (os.x - r.o.x) * r.dinv.x, cy = (os.y - r.o.y) * r.dinv.y, cz = (os.z - r.o.z) * r.dinv.z;
-        const float sx = os.w * r.dinv.x, sy = os.w * r.dinv.y, sz = os.w * r.dinv.z;
-        AxisT tx, ty, tz;
-        if (s.bvh1) {
-            // the ray's time clamped to the shutter, as the transforms are
-            const float t = fminf(fmaxf(r.time, 0.0f), 1.0f);
-            tx = axis_t_moving(px, axis_planes(nd.delta[0], ds0), t, sx, cx);
-            ty = axis_t_moving(py, axis_planes(nd.delta[1], ds1), t, sy, cy);
-            tz = axis_t_moving(pz, axis_planes(nd.delta[2], ds2), t, sz, cz);
-        } else {
-            tx = axis_t(px, sx, cx);
-            ty = axis_t(py, sy, cy);
-            tz = axis_t(pz, sz, cz);
-        }
-        // BBox4::intersect_ray lanes (basics/bbox.hpp:566-595) for distances
-        // in range (no NaN); keys are the near distances of hit children,
-        // +inf otherwise
+        float4 nx, fx, ny, fy, nz, fz;
+        node_boxes(s, ref, r.time, ds0, ds1, ds2, nx, fx, ny, fy, nz, fz);
+        const int4 ch = reinterpret_cast<const int4*>(s.bvh + ref)[6];
+        // BBox4::intersect_ray lanes (basics/bbox.hpp:566-595) for a finite
+        // inverse direction (no NaN); keys are the near distances of hit
+        // children, +inf otherwise
 #define PSY_LANE(LN, KEY)                                                                            \
     float KEY;                                                                                       \
     {                                                                                                \
-        const float mins = fmaxf(fmaxf(tx.n[LN], ty.n[LN]), fmaxf(tz.n[LN], 0.0f)) * PSY_NODE_NEAR;  \
-        const float maxs = fminf(fminf(tx.f[LN], ty.f[LN]), tz.f[LN]) * PSY_NODE_FAR;                \
+        const float xlo = (nx.LN - r.o.x) * r.dinv.x;                                                \
+        const float xhi = (fx.LN - r.o.x) * r.dinv.x;                                                \
+        const float ylo = (ny.LN - r.o.y) * r.dinv.y;                                                \
+        const float yhi = (fy.LN - r.o.y) * r.dinv.y;                                                \
+        const float zlo = (nz.LN - r.o.z) * r.dinv.z;                                                \
+        const float zhi = (fz.LN - r.o.z) * r.dinv.z;                                                \
+        const float mins = fmaxf(fmaxf(xlo, ylo), fmaxf(zlo, 0.0f));                                 \
+        const float maxs = fminf(fminf(xhi, yhi), zhi) * PSY_BBOX_MAXT_ADJUST;                       \
         KEY = ((mins < L.b.t) && (mins <= maxs)) ? mins : INFINITY;                                  \
     }
-        PSY_LANE(0, k0)
-        PSY_LANE(1, k1)
-        PSY_LANE(2, k2)
-        PSY_LANE(3, k3)
+        PSY_LANE(x, k0)
+        PSY_LANE(y, k1)
+        PSY_LANE(z, k2)
+        PSY_LANE(w, k3)
 #undef PSY_LANE
         int32_t r0 = ch.x, r1 = ch.y, r2 = ch.z, r3 = ch.w;
         cmpswap(k0, r0, k1, r1);
