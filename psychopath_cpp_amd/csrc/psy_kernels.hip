@@ -775,8 +775,7 @@ template <bool W, int S>
 static void launch_deep(const DevScene& s, const float* rays, int64_t n, int64_t rs, const DevHits& h, uint32_t flags,
                         const uint32_t* queue, const uint32_t* heads, const uint32_t* pool, uint32_t* counters,
                         const TraceTuning& tune, hipStream_t st) {
-    // a wave per ray, of which a call hands on few
-    const unsigned blocks = (unsigned)std::min<int64_t>((n + 7) / 8, DEEP_ROUND);
+    const unsigned blocks = coop_blocks(n);
     uint32_t* coop_queue = const_cast<uint32_t*>(queue) + n;
     const int32_t budget = std::max<int32_t>(1, tune.deep_budget);
     if (n >= (int64_t)tune.wide_min) {

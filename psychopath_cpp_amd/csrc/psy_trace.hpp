@@ -822,15 +822,24 @@ constexpr int TRACE_BLOCK = PSY_TRACE_BLOCK;  // threads per block of the trace 
 // for the few rays a primary stream hands on.  Longer queues are worked a
 // lane per ray (k_trace_deep, 2 waves per SIMD: 256 VGPRs, paid for with
 // spills), and k_trace_coop follows as the third pass, over the rays that
-// outran a lane's limits.  wide_min is k_trace_coop's number of waves by
-// default, so that none of them takes one ray after another.  (Until it
-// worked on lists, short queues had a second build of k_trace_deep at 1 wave
-// per SIMD: the object stream of 2^22 rays is the same within 0.3 %, the
-// heightfield crop at 331x173x3, 8 calls of a few queued rays, 3.49 ms for
-// 3.65.)  Each form launches one resident round of 64-thread blocks over 256
-// CUs.  wide_min and the second pass's node budget are launch parameters.
+// outran a lane's limits.  wide_min is by default the waves of
+// k_trace_coop's resident round (DEEP_ROUND), from where it would take one
+// ray after another.  Until it worked on lists, queues shorter than 4096
+// had a build of k_trace_deep at 1 wave per SIMD; camera rays over the
+// heightfield diced 4 levels deep, all of them queued: 1000 rays 747 us
+// then, 248 now, 1500 759 and 625, 4000 877 and 740.  Each form launches at
+// most one resident round of 64-thread blocks over 256 CUs.  wide_min and
+// the second pass's node budget are launch parameters.
 constexpr int DEEP_WIDE_WAVES = 2;
 constexpr int DEEP_ROUND = 1024;          // blocks per wave per SIMD over 256 CUs
+// Blocks of k_trace_coop for a call of n rays: any of its rays may be
+// queued, and a queue shorter than wide_min has no other kernel.  With an
+// eighth of them, a short call that queues most of its rays worked up to 8
+// in a row on one wave: 1024 rays through 4096 nested spheres (588 queued)
+// 24.5 ms, now 8.1; 1000 over the heightfield above 402 us, now 248.  A
+// call that queues none pays about 1 us for the waves that find no ray
+// (6144 rays 60.5 us, now 61.5).
+inline unsigned coop_blocks(int64_t n) { return (unsigned)std::min<int64_t>(n, DEEP_ROUND); }
 
 // A ray of the stream: world form (PSY_WRAY_PLANES, footprint derived here,
 // basics/ray.hpp:310-323) or object form (PSY_RAY_PLANES).

@@ -49,6 +49,8 @@ def lib():
                                    C.c_int, vp, vp, vp, C.POINTER(i64), C.c_int]
     L.hb_set_spectrum_grid.argtypes = [vp, C.c_int, C.c_int, vp, C.c_int, C.c_int, C.c_float, C.c_float, vp]
     L.hb_scene_stack_need.argtypes = [C.POINTER(abi.SceneDesc), C.c_int, C.POINTER(C.c_int)]
+    L.hb_second_pass_waves.argtypes = [i64]
+    L.hb_second_pass_waves.restype = i64
     _lib = L
     return L
 

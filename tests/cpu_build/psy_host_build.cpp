@@ -129,6 +129,9 @@ int hb_scene_stack_need(const psy_scene_desc* d, int dice_depth, int* need) {
     return rc;
 }
 
+// Waves of the second pass's wave-per-ray kernel in a call of n rays.
+int64_t hb_second_pass_waves(int64_t n) { return (int64_t)coop_blocks(n) * (TRACE_BLOCK / 64); }
+
 // psy_trace_world / psy_trace_rays on the CPU.  Returns a psy_status;
 // *retraced = rays that took the second pass.
 int hb_trace(const psy_scene_desc* d, int dice_depth, int world, const float* rays, int64_t n, uint32_t flags,
