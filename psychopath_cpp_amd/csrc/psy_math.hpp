@@ -289,21 +289,7 @@ PSY_HD RayW ray_widths(V3 o, V3 d, V3 odx, V3 ody, V3 ddx, V3 ddy) {
     else { w.dwy = (ly - w.owy) / tdy; w.fwy = ly; }
     return w;
 }
-// Ray::min_width with its two flip distances precomputed (they depend on
-// the footprint only): min_width(r, a, b) == min_width_flip(r, flip_x(r),
-// flip_y(r), a, b) bit for bit.
-PSY_HD float flip_x(const RayW& r) { return (r.owx - r.fwx) / r.dwx; }
-PSY_HD float flip_y(const RayW& r) { return (r.owy - r.fwy) / r.dwy; }
-PSY_HD float min_width_flip(const RayW& r, float tflipx, float tflipy, float tnear, float tfar) {
-    float minx, miny;
-    if (tnear < tflipx && tfar > tflipx) minx = r.fwx;
-    else minx = smin(fabsf((r.owx - r.fwx) + (r.dwx * tnear)) + r.fwx,
-                     fabsf((r.owx - r.fwx) + (r.dwx * tfar)) + r.fwx);
-    if (tnear < tflipy && tfar > tflipy) miny = r.fwy;
-    else miny = smin(fabsf((r.owy - r.fwy) + (r.dwy * tnear)) + r.fwy,
-                     fabsf((r.owy - r.fwy) + (r.dwy * tfar)) + r.fwy);
-    return smin(minx, miny);
-}
+// Ray::min_width
 PSY_HD float min_width(const RayW& r, float tnear, float tfar) {
     const float tflipx = (r.owx - r.fwx) / r.dwx;
     const float tflipy = (r.owy - r.fwy) / r.dwy;

@@ -992,7 +992,7 @@ constexpr int persist_waves(bool world, int stack) { return stack <= 16 ? PSY_PE
 
 // A ray footprint as the walk uses it: per axis the width at t is
 // |k + dw t| + fw, except fw on an interval that holds the flip distance
-// (min_width_flip, with k = ow - fw).
+// (min_width, with k = ow - fw).
 struct Foot { float kx, ky, dwx, dwy, fwx, fwy, flx, fly; };
 
 struct Lane {
@@ -1142,25 +1142,38 @@ struct RayStream {
     }
 };
 
-// The walk's form of a footprint; false for one with an infinite term, whose
-// widths can be NaN at some distances only (the second pass follows the
-// reference there).  A footprint that is NaN on an axis makes the width NaN,
-// which dices to min_upoly (dice_width), as a width of 0 does; std::min
-// passes a NaN on when x has it and ignores it in y.
-PSY_DEV bool make_foot(const RayW& w, Foot& f) {
+// One axis of the walk's form of a footprint.  Its width at t is
+// |k + d t| + f, or f on an interval that holds the flip distance `fl`; with
+// an infinite k (a caller's "do not dice") that is infinite everywhere, as it
+// should be.  What the form above would get wrong is replaced by what the
+// reference's std::min sequence makes of it: a width that is NaN everywhere
+// dices to min_upoly (dice_width) if it is x's, as a width of 0 does, and is
+// ignored if it is y's, as an infinite one is.  A width with an infinite d is
+// infinite but at t = 0, where it is NaN: the flip distance 2^-149 tells that
+// distance from all others.
+template <bool Y>
+PSY_DEV void foot_odd_axis(float& k, float& d, float& f, float& fl) {
+    const bool opposed = fabsf(k) == INFINITY && fabsf(d) == INFINITY && (k < 0.0f) != (d < 0.0f);
+    const bool nan = k != k || d != d || f == -INFINITY || opposed;
+    const bool inf = !nan && fabsf(d) == INFINITY;
+    k = nan ? 0.0f : inf ? INFINITY : k;
+    d = nan || inf ? 0.0f : d;
+    f = nan ? (Y ? INFINITY : 0.0f) : inf ? 0.0f : f;
+    fl = nan || (Y && inf) ? INFINITY : inf ? u2f(1u) : fl;
+}
+PSY_DEV void make_foot(const RayW& w, Foot& f) {
     f.kx = w.owx - w.fwx; f.dwx = w.dwx; f.fwx = w.fwx;
     f.ky = w.owy - w.fwy; f.dwy = w.dwy; f.fwy = w.fwy;
-    f.flx = flip_x(w);
-    f.fly = flip_y(w);
-    const bool nan_x = w.owx != w.owx || w.dwx != w.dwx || w.fwx != w.fwx;
-    const bool nan_y = w.owy != w.owy || w.dwy != w.dwy || w.fwy != w.fwy;
-    if (nan_x) { f.kx = f.dwx = f.fwx = 0.0f; f.flx = INFINITY; }
-    if (nan_y) { f.ky = f.dwy = 0.0f; f.fwy = INFINITY; f.fly = INFINITY; }
-    return finite3(mk(f.kx, f.dwx, f.fwx)) && finite3(mk(f.ky, f.dwy, nan_y ? 0.0f : f.fwy));
+    f.flx = f.kx / f.dwx;
+    f.fly = f.ky / f.dwy;
+    if (!(finite3(mk(f.kx, f.dwx, f.fwx)) && finite3(mk(f.ky, f.dwy, f.fwy)))) {
+        foot_odd_axis<false>(f.kx, f.dwx, f.fwx, f.flx);
+        foot_odd_axis<true>(f.ky, f.dwy, f.fwy, f.fly);
+    }
 }
 
-// min_width_flip over a box's near and far distance for a make_foot footprint
-// and a box that is hit (near is finite and not below 0; a far distance of
+// min_width over a box's near and far distance for a make_foot footprint and
+// a box that is hit (near is finite and not below 0; a far distance of
 // infinity times a dw of 0 is ignored by fminf as by std::min).
 PSY_DEV float foot_width(const Foot& f, float h0, float h1) {
     float wx = fminf(fabsf(f.kx + f.dwx * h0), fabsf(f.kx + f.dwx * h1)) + f.fwx;
@@ -1201,9 +1214,8 @@ PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i) {
     L.wframe = -1;  // read by world rays only
     // the main pass's box tests assume a finite inverse direction; the
     // second pass follows the reference's NaN behaviour exactly
-    bool plain = finite3(L.r.dinv);
-    if (!WORLD) plain = make_foot(L.r.w, L.foot) && plain;
-    if (!plain) {
+    if (!WORLD) make_foot(L.r.w, L.foot);
+    if (!finite3(L.r.dinv)) {
         L.state = LANE_RETRACE;
         L.next = CHILD_EMPTY;
     }
@@ -1211,7 +1223,7 @@ PSY_DEV void lane_start(const DevScene& s, Lane& L, float max_t, uint32_t i) {
 
 // The patch-space ray of a walk through leaf I's split tree (world rays:
 // through the leaf's transform at the ray's time) and its footprint; false
-// when its inverse direction or its footprint is not finite.  They depend
+// when its inverse direction is not finite.  They depend
 // on the leaf's transforms alone, so the patches of one instance (a
 // subdivision surface's, an instanced assembly's) reuse them: a ray that
 // meets several patches of a transformed instance derives them once.
@@ -1233,9 +1245,10 @@ PSY_DEV bool walk_ray(const DevScene& s, Lane& L, const DevInstance& I, const Sr
         ddx = m_dir(x, ddx);
         ddy = m_dir(x, ddy);
     }
-    const bool plain = make_foot(ray_widths(L.wo, d, odx, ody, ddx, ddy), L.foot) && finite3(L.wdinv);
-    L.wframe = plain ? frame : -1;
-    return plain;
+    make_foot(ray_widths(L.wo, d, odx, ody, ddx, ddy), L.foot);
+    const bool finite = finite3(L.wdinv);
+    L.wframe = finite ? frame : -1;
+    return finite;
 }
 
 // One unit of work; true when the ray is finished (or must be retraced).

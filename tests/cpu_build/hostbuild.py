@@ -49,6 +49,8 @@ def lib():
                                    C.c_int, vp, vp, vp, C.POINTER(i64), C.c_int]
     L.hb_set_spectrum_grid.argtypes = [vp, C.c_int, C.c_int, vp, C.c_int, C.c_int, C.c_float, C.c_float, vp]
     L.hb_scene_stack_need.argtypes = [C.POINTER(abi.SceneDesc), C.c_int, C.POINTER(C.c_int)]
+    L.hb_foot_mismatches.argtypes = [vp, C.c_int, vp, C.c_int, vp, C.c_int, C.c_float, C.c_float, vp]
+    L.hb_foot_mismatches.restype = i64
     L.hb_second_pass_waves.argtypes = [i64]
     L.hb_second_pass_waves.restype = i64
     _lib = L
@@ -75,6 +77,15 @@ def trace(scene_py, rays, world=True, dice_depth=10, occlusion_only=False, threa
     if rc != 0:
         raise RuntimeError(f"hb_trace failed with status {rc}")
     return {"t": t, "inst": inst, "u": u, "v": v, "aux": aux, "retraced": rt.value}
+
+
+def foot_mismatches(values, intervals, sizes, rate, min_upoly):
+    """(count, first) of the footprints made of `values` whose size test in the main pass and in the second
+    pass differ on one of the (near, far) intervals and node sizes."""
+    v, h, z = (np.ascontiguousarray(x, np.float32) for x in (values, intervals, sizes))
+    first = np.zeros(6, np.float32)
+    bad = lib().hb_foot_mismatches(_p(v), v.size, _p(h), h.size // 2, _p(z), z.size, rate, min_upoly, _p(first))
+    return bad, first
 
 
 def scene_stack_need(scene_py, dice_depth=0):

@@ -132,6 +132,34 @@ int hb_scene_stack_need(const psy_scene_desc* d, int dice_depth, int* need) {
 // Waves of the second pass's wave-per-ray kernel in a call of n rays.
 int64_t hb_second_pass_waves(int64_t n) { return (int64_t)coop_blocks(n) * (TRACE_BLOCK / 64); }
 
+// Footprints (ow, dw, fw per axis from the n values, all n^6 of them) on
+// which the main pass's size test (foot_width) and the second pass's
+// (min_width, as the reference has it) decide differently for some of the
+// n_h box intervals (near, far) and n_s node sizes; `first` gets the first.
+int64_t hb_foot_mismatches(const float* v, int n, const float* h, int n_h, const float* sizes, int n_s, float rate,
+                           float min_upoly, float* first) {
+    int64_t bad = 0;
+    int64_t total = 1;
+    for (int k = 0; k < 6; ++k) total *= n;
+    for (int64_t c = 0; c < total; ++c) {
+        float x[6];
+        int64_t r = c;
+        for (int k = 0; k < 6; ++k, r /= n) x[k] = v[r % n];
+        const RayW w{x[0], x[1], x[2], x[3], x[4], x[5]};
+        Foot f;
+        make_foot(w, f);
+        bool same = true;
+        for (int j = 0; j < n_h; ++j) {
+            const float a = dice_width(min_width(w, h[2 * j], h[2 * j + 1]) * rate, min_upoly);
+            const float b = foot_width(f, h[2 * j], h[2 * j + 1]) * rate;
+            for (int q = 0; q < n_s; ++q) same = same && (sizes[q] <= a) == (sizes[q] <= b || sizes[q] <= min_upoly);
+        }
+        if (!same && bad++ == 0)
+            for (int k = 0; k < 6; ++k) first[k] = x[k];
+    }
+    return bad;
+}
+
 // psy_trace_world / psy_trace_rays on the CPU.  Returns a psy_status;
 // *retraced = rays that took the second pass.
 int hb_trace(const psy_scene_desc* d, int dice_depth, int world, const float* rays, int64_t n, uint32_t flags,

@@ -59,3 +59,33 @@ def test_footprints_that_are_not_finite(plane, value):
     b = hostbuild.trace(sc, rays, world=False, dice_depth=0)
     for k in ("t", "inst", "u", "v", "aux"):
         assert np.array_equal(a[k], b[k]), k
+
+
+# ow dw fw of one axis or both, as a caller may set them to mean "do not dice" (ow, dw), or by accident
+@pytest.mark.parametrize("planes", [(8, 9), (10, 11), (8, 9, 10, 11), (12, 13), (8, 9, 10, 11, 12, 13), (8,), (9,), (10,), (11,)])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_footprints_that_are_not_finite_stay_in_the_main_pass(planes, value):
+    rays = _object_rays(60, 0.05)
+    rays[10:12] = 0.01
+    for p in planes:
+        rays[p] = value
+    rays[2, ::2] = 0.05  # half of them start inside the patch's box
+    sc = _scene("bilinear", min_upoly=0.02)
+    a = hostbuild.trace(sc, rays, world=False, dice_depth=14)
+    b = hostbuild.trace(sc, rays, world=False, dice_depth=0)
+    assert a["retraced"] == 0  # the cache reaches min_upoly
+    assert (a["inst"] == 0).sum() > 10
+    for k in ("t", "inst", "u", "v", "aux"):
+        assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("rate", [0.25, 1.0])
+@pytest.mark.parametrize("min_upoly", [0.0, 1e-5, 0.5])
+def test_size_test_is_the_references_for_every_footprint(rate, min_upoly):
+    """Intervals that end after the ray's origin (no hit lies in another)."""
+    inf = np.inf
+    bad, first = hostbuild.foot_mismatches(
+        [0.0, 0.3, 0.01, -1.0, 1e38, inf, -inf, np.nan],
+        [(0, 1), (0.5, 2), (0, inf), (3, inf), (1e-30, 1e-20), (1e-42, 1e-3), (2, 2)], [0.0, 1e-6, 0.4, 1e30], rate,
+        min_upoly)
+    assert bad == 0, first
