@@ -286,8 +286,9 @@ int psy_ctx_set_render_chunk(psy_ctx* ctx, int64_t paths);
  * chunk's short late bounces run beside the others' work.  The caller's
  * stream waits for all of them at the end.  While such a render runs, the
  * calling thread polls the chunks' events (one host core stays busy).
- * Where memory is short a render takes fewer, down to 2.  Same samples as
- * with 1. */
+ * A chunk after the second is taken only where its buffers leave a sixteenth
+ * of the device's memory free, and a render that runs out of memory goes on
+ * with two.  Same samples as with 1. */
 int psy_ctx_set_render_streams(psy_ctx* ctx, int streams);
 /* Register budget of PSY_RENDER_WAVEFRONT's shading kernel for the steps
  * that take a hit and sample a light (no counterpart in the reference):

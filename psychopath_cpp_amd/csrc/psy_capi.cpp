@@ -150,25 +150,30 @@ void gtr_validate(float roughness, float tail_shape, float fresnel, DevShader& o
     o.norm = (float)((double)top / bottom);
 }
 
-int ensure_trace_scratch(DBuf& queue, DBuf& counters, int64_t& queue_cap, int64_t n) {
-    if (!counters.p) {
-        int rc = counters.alloc(sizeof(uint32_t) * 8);
-        if (rc) return rc;
-    }
-    if (n <= queue_cap) return PSY_OK;
-    HIP_OK(hipDeviceSynchronize());
-    queue.release();
-    const int64_t cap = std::max<int64_t>(n, 1 << 16);
+static int64_t trace_scratch_cap(int64_t n) { return std::max<int64_t>(n, 1 << 16); }
+
+size_t trace_scratch_bytes(int64_t n) {
     // for up to cap rays: the second pass's queue, the third pass's queue,
     // the second-pass rays' deep-node lists and the deep-node pool (3 words
     // an entry), then the main pass's continuation buffer
-    int rc = queue.alloc((size_t)(6 * cap + psy::cont_area_words(cap)) * sizeof(uint32_t));
-    if (rc) { queue_cap = 0; return rc; }
-    queue_cap = cap;
-    return PSY_OK;
+    const int64_t cap = trace_scratch_cap(n);
+    return (size_t)(6 * cap + cont_area_words(cap)) * sizeof(uint32_t);
 }
 
-int ensure_queue(psy_ctx* ctx, int64_t n) { return ensure_trace_scratch(ctx->queue, ctx->counters, ctx->queue_cap, n); }
+hipError_t try_trace_scratch(DBuf& queue, DBuf& counters, int64_t& queue_cap, int64_t n) {
+    if (!counters.p)
+        if (const hipError_t e = counters.try_alloc(sizeof(uint32_t) * 8)) return e;
+    if (n <= queue_cap) return hipSuccess;
+    if (const hipError_t e = hipDeviceSynchronize()) return e;
+    queue_cap = 0;
+    if (const hipError_t e = queue.try_alloc(trace_scratch_bytes(n))) return e;
+    queue_cap = trace_scratch_cap(n);
+    return hipSuccess;
+}
+
+int ensure_queue(psy_ctx* ctx, int64_t n) {
+    return alloc_status(try_trace_scratch(ctx->queue, ctx->counters, ctx->queue_cap, n));
+}
 
 static int capturing(hipStream_t st, bool* yes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;

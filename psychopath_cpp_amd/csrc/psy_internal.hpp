@@ -24,6 +24,11 @@ int floats_per_kind(int kind);
             return ::psy::fail(PSY_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
+// The status, with its message, of an allocation that returned `e`.
+inline int alloc_status(hipError_t e) {
+    return e == hipSuccess ? PSY_OK : fail(PSY_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
+}
+
 // Owning device allocation.
 struct DBuf {
     void* p = nullptr;
@@ -37,20 +42,23 @@ struct DBuf {
         p = nullptr;
         bytes = 0;
     }
-    int alloc(size_t b) {
+    // on failure nothing is held, and no HIP error is left behind
+    hipError_t try_alloc(size_t b) {
         release();
-        bytes = b;
-        if (b == 0) return 0;
-        hipError_t e = hipMalloc(&p, b);
+        if (b == 0) return hipSuccess;
+        const hipError_t e = hipMalloc(&p, b);
         if (e != hipSuccess) {
             p = nullptr;
-            bytes = 0;
-            return fail(PSY_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
+            (void)hipGetLastError();
+        } else {
+            bytes = b;
         }
-        return 0;
+        return e;
     }
+    int alloc(size_t b) { return alloc_status(try_alloc(b)); }
     // grows (never shrinks) to at least b bytes; contents are not kept
-    int reserve(size_t b) { return b <= bytes && p ? 0 : alloc(b); }
+    hipError_t try_reserve(size_t b) { return b <= bytes && p ? hipSuccess : try_alloc(b); }
+    int reserve(size_t b) { return alloc_status(try_reserve(b)); }
     int upload(const void* src, size_t b) {
         int rc = alloc(b);
         if (rc) return rc;
@@ -283,7 +291,39 @@ void make_halton_tables(std::vector<HaltonDim>& dims, std::vector<uint16_t>& per
 // Grows the context's trace scratch (second-pass queue) to n rays.
 int ensure_queue(psy_ctx* ctx, int64_t n);
 // The same for a given queue / counters pair and its capacity in rays.
-int ensure_trace_scratch(DBuf& queue, DBuf& counters, int64_t& queue_cap, int64_t n);
+hipError_t try_trace_scratch(DBuf& queue, DBuf& counters, int64_t& queue_cap, int64_t n);
+// Bytes of a trace scratch for n rays.
+size_t trace_scratch_bytes(int64_t n);
+
+// Chunks a render takes in flight, of `want`: each after the second only if
+// what its buffers lack (lacks[k] bytes) leaves a sixteenth of the device's
+// memory free for the rest of the program, which may well allocate between
+// two renders and had that memory while two chunks were the default.
+inline int slots_that_fit(int want, const int64_t* lacks, int64_t free_bytes, int64_t total_bytes) {
+    int64_t left = free_bytes - total_bytes / 16;
+    int n = 0;
+    for (; n < want; ++n) {
+        if (n >= 2 && lacks[n] > 0 && lacks[n] > left) break;
+        left -= lacks[n];
+    }
+    return n;
+}
+
+// Allocates for `slots` chunks in flight through take(slots) or, when that
+// runs out of memory, for the first two at most, once drop(slots) has freed
+// what chunks beyond them hold (true: it has freed something).  Any other
+// error is returned as it is.
+template <class Take, class Drop>
+hipError_t take_slots(int& slots, Take take, Drop drop) {
+    for (;;) {
+        const hipError_t e = take(slots);
+        if (e != hipErrorOutOfMemory) return e;
+        const int fewer = slots < 2 ? slots : 2;
+        const bool freed = drop(fewer);
+        if (fewer == slots && !freed) return e;
+        slots = fewer;
+    }
+}
 // Orders a call that uses the context's trace scratch on stream st after
 // the previous such call (made on any stream): scratch_order before the
 // call's first launch, scratch_release after its last.  Streams under graph

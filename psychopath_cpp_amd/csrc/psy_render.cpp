@@ -441,35 +441,64 @@ float* carve_slot(float* base, int64_t cap, bool own_samples, RenderBuffers& B, 
     return *samples + (own_samples ? 3 * cap : 0);
 }
 
-// After plan_render: the scratch, with `extra_floats` after the render's
-// own, and that of chunks 1..U.slots-1.
-int alloc_render(psy_ctx* ctx, bool own_samples, int64_t extra_floats, RenderSetup& U) {
+// After plan_render: the scratch, with `extra` floats and `slot_extra` for
+// each chunk in flight after the render's own, and that of chunks
+// 1..U.slots-1.  Where memory is short, U.slots falls, to 2 at least.
+int alloc_render(psy_ctx* ctx, bool own_samples, int64_t extra, int64_t slot_extra, RenderSetup& U) {
     const int64_t cap = U.cap;
     if (cap > (int64_t)INT32_MAX) return fail(PSY_ERR_UNSUPPORTED, "psy_render: more than 2^31 paths per chunk");
-    const int64_t f_slot = slot_floats(cap, own_samples);
-    const int64_t f_extra = (extra_floats + 63) / 64 * 64;
-    if (int rc = ctx->render_scratch.reserve((size_t)(f_slot + f_extra) * sizeof(float))) return rc;
-    if (int rc = ensure_queue(ctx, cap)) return rc;
+    const size_t slot_bytes = (size_t)slot_floats(cap, own_samples) * sizeof(float);
+    auto main_bytes = [&](int slots) {
+        return slot_bytes + (size_t)((extra + slots * slot_extra + 63) / 64 * 64) * sizeof(float);
+    };
+    auto lack = [](const DBuf& b, size_t need) { return need > b.bytes ? (int64_t)(need - b.bytes) : (int64_t)0; };
+    // a render that needs no memory asks for none, and for nothing about it
+    int64_t lacks[psy_ctx::MAX_RENDER_SLOTS] = {}, more = 0;
+    for (int k = 0; k < U.slots; ++k) {
+        lacks[k] = lack(ctx->render_scratch, main_bytes(k + 1)) - (k > 0 ? lack(ctx->render_scratch, main_bytes(k)) : 0);
+        if (k == 0 && cap > ctx->queue_cap) lacks[k] += lack(ctx->queue, trace_scratch_bytes(cap));
+        if (k > 0) lacks[k] += lack(ctx->slot_scratch[k - 1], slot_bytes);
+        if (k > 0 && cap > ctx->slot_queue_cap[k - 1]) lacks[k] += lack(ctx->slot_queue[k - 1], trace_scratch_bytes(cap));
+        if (k >= 2) more += lacks[k];
+    }
+    if (more > 0) {
+        size_t free_bytes = 0, total_bytes = 0;
+        HIP_OK(hipMemGetInfo(&free_bytes, &total_bytes));
+        U.slots = slots_that_fit(U.slots, lacks, (int64_t)free_bytes, (int64_t)total_bytes);
+    }
+    const hipError_t e = take_slots(
+        U.slots,
+        [&](int slots) {
+            hipError_t r = ctx->render_scratch.try_reserve(main_bytes(slots));
+            if (!r) r = try_trace_scratch(ctx->queue, ctx->counters, ctx->queue_cap, cap);
+            for (int k = 0; k + 1 < slots && !r; ++k) {
+                r = ctx->slot_scratch[k].try_reserve(slot_bytes);
+                if (!r) r = try_trace_scratch(ctx->slot_queue[k], ctx->slot_counters[k], ctx->slot_queue_cap[k], cap);
+            }
+            return r;
+        },
+        [&](int slots) {
+            bool freed = false;
+            (void)hipDeviceSynchronize();  // an earlier render may still use them
+            for (int k = std::max(0, slots - 1); k + 1 < psy_ctx::MAX_RENDER_SLOTS; ++k) {
+                freed = freed || ctx->slot_scratch[k].p || ctx->slot_queue[k].p;
+                ctx->slot_scratch[k].release();
+                ctx->slot_queue[k].release();
+                ctx->slot_queue_cap[k] = 0;
+            }
+            return freed;
+        });
+    if (e != hipSuccess) return alloc_status(e);
     U.extra = carve_slot((float*)ctx->render_scratch.p, cap, own_samples, U.B, &U.chunk_samples);
     if (!ctx->host_counts)
         HIP_OK(hipHostMalloc((void**)&ctx->host_counts, 16 * psy_ctx::MAX_RENDER_SLOTS * sizeof(uint32_t),
                              hipHostMallocDefault));
     if (U.slots > 1) {
         if (!ctx->render_join) HIP_OK(hipEventCreateWithFlags(&ctx->render_join, hipEventDisableTiming));
-        for (hipEvent_t& e : ctx->render_done)
-            if (!e) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        for (hipEvent_t& ev : ctx->render_done)
+            if (!ev) HIP_OK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
     }
     for (int k = 0; k + 1 < U.slots; ++k) {
-        int rc = ctx->slot_scratch[k].reserve((size_t)f_slot * sizeof(float));
-        if (!rc) rc = ensure_trace_scratch(ctx->slot_queue[k], ctx->slot_counters[k], ctx->slot_queue_cap[k], cap);
-        if (rc && k >= 1) {
-            // no memory for a third or fourth chunk: go on with those there are
-            (void)hipGetLastError();
-            ctx->slot_scratch[k].release();
-            U.slots = k + 1;
-            break;
-        }
-        if (rc) return rc;
         if (!ctx->slot_stream[k]) HIP_OK(hipStreamCreateWithFlags(&ctx->slot_stream[k], hipStreamNonBlocking));
         carve_slot((float*)ctx->slot_scratch[k].p, cap, own_samples, U.Bx[k], &U.samples_x[k]);
     }
@@ -784,11 +813,11 @@ int render_forms(psy_ctx* ctx, const psy_scene* s, const psy_render_params* prm,
             window = std::min(U.total, std::max<int64_t>(4 * U.cap, (int64_t)1 << 26));
             window = std::max<int64_t>(U.spp, window / U.spp * U.spp);
         }
-        if (int rc = alloc_render(ctx, false, 64 + U.cap + (sample_xyz ? 0 : 3 * window), U)) return rc;
+        if (int rc = alloc_render(ctx, false, 64 + U.cap + (sample_xyz ? 0 : 3 * window), 0, U)) return rc;
         return run_stream(ctx, s, prm, R, U, window, film_xyz, sample_xyz, rays_traced, st);
     }
     if (ctx->render_mode == PSY_RENDER_WAVEFRONT) U.slots = render_slots(ctx, U);
-    if (int rc = alloc_render(ctx, sample_xyz == nullptr, 0, U)) return rc;
+    if (int rc = alloc_render(ctx, sample_xyz == nullptr, 0, 0, U)) return rc;
     if (ctx->render_mode == PSY_RENDER_FUSED) return run_fused(ctx, s, prm, R, U, film_xyz, sample_xyz, rays_traced, st);
     return run_wavefront(ctx, s, prm, R, U, film_xyz, sample_xyz, nullptr, rays_traced, st);
 }
@@ -1047,13 +1076,7 @@ int psy_adjoint(psy_ctx* ctx, const psy_scene* s, const psy_render_params* prm, 
     const int64_t f_q = (int64_t)ADJ_STATE_PLANES * U.cap;
     const int64_t f_grad = (n_params + 63) / 64 * 64;
     const int64_t f_part = J.lds ? (int64_t)J.rows * n_params : 0;
-    int rc_alloc = alloc_render(ctx, true, U.slots * (f_q + f_part) + f_grad, U);
-    if (rc_alloc && U.slots > 2) {  // with less memory, two chunks
-        (void)hipGetLastError();
-        U.slots = 2;
-        rc_alloc = alloc_render(ctx, true, U.slots * (f_q + f_part) + f_grad, U);
-    }
-    if (rc_alloc) return rc_alloc;
+    if (int rc = alloc_render(ctx, true, f_grad, f_q + f_part, U)) return rc;
     J.q = U.extra;
     J.grad = J.q + U.slots * f_q;
     J.partials = J.grad + f_grad;

@@ -51,6 +51,9 @@ def lib():
     L.hb_scene_stack_need.argtypes = [C.POINTER(abi.SceneDesc), C.c_int, C.POINTER(C.c_int)]
     L.hb_foot_mismatches.argtypes = [vp, C.c_int, vp, C.c_int, vp, C.c_int, C.c_float, C.c_float, vp]
     L.hb_foot_mismatches.restype = i64
+    L.hb_take_slots.argtypes = [C.c_int, C.c_int, C.POINTER(C.c_int), C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int),
+                                C.POINTER(C.c_int)]
+    L.hb_slots_that_fit.argtypes = [C.c_int, C.POINTER(i64), i64, i64]
     L.hb_second_pass_waves.argtypes = [i64]
     L.hb_second_pass_waves.restype = i64
     _lib = L
@@ -77,6 +80,18 @@ def trace(scene_py, rays, world=True, dice_depth=10, occlusion_only=False, threa
     if rc != 0:
         raise RuntimeError(f"hb_trace failed with status {rc}")
     return {"t": t, "inst": inst, "u": u, "v": v, "aux": aux, "retraced": rt.value}
+
+
+def take_slots(want, need, held, room, error=0):
+    """(status, chunks in flight, attempts) of a render's allocation: see hb_take_slots."""
+    slots, asked = C.c_int(), C.c_int()
+    rc = lib().hb_take_slots(want, need, (C.c_int * len(held))(*held), len(held), room, error, C.byref(slots),
+                             C.byref(asked))
+    return rc, slots.value, asked.value
+
+
+def slots_that_fit(want, lacks, free_bytes, total_bytes):
+    return lib().hb_slots_that_fit(want, (C.c_int64 * len(lacks))(*lacks), free_bytes, total_bytes)
 
 
 def foot_mismatches(values, intervals, sizes, rate, min_upoly):

@@ -132,6 +132,48 @@ int hb_scene_stack_need(const psy_scene_desc* d, int dice_depth, int* need) {
 // Waves of the second pass's wave-per-ray kernel in a call of n rays.
 int64_t hb_second_pass_waves(int64_t n) { return (int64_t)coop_blocks(n) * (TRACE_BLOCK / 64); }
 
+// A render's memory, in units: room for `room`, of which chunks beyond the
+// first hold held[k] from an earlier render and every chunk of this one needs
+// `need`.  Returns the hipError_t, the chunks it got and how often it asked.
+int hb_take_slots(int want, int need, const int* held, int n_held, int room, int error, int* slots, int* asked) {
+    std::vector<int> have(held, held + n_held);
+    have.resize(8, 0);
+    int own = 0;
+    *slots = want;
+    *asked = 0;
+    auto used = [&]() {
+        int u = own;
+        for (int x : have) u += x;
+        return u;
+    };
+    return (int)take_slots(
+        *slots,
+        [&](int n) {
+            ++*asked;
+            if (error) return (hipError_t)error;
+            if (used() - own + need > room) return hipErrorOutOfMemory;
+            own = need;
+            for (int k = 0; k + 1 < n; ++k) {
+                if (have[k] >= need) continue;
+                if (used() - have[k] + need > room) return hipErrorOutOfMemory;
+                have[k] = need;
+            }
+            return hipSuccess;
+        },
+        [&](int n) {
+            bool freed = false;
+            for (size_t k = (size_t)std::max(0, n - 1); k < have.size(); ++k) {
+                freed = freed || have[k] > 0;
+                have[k] = 0;
+            }
+            return freed;
+        });
+}
+
+int hb_slots_that_fit(int want, const int64_t* lacks, int64_t free_bytes, int64_t total_bytes) {
+    return slots_that_fit(want, lacks, free_bytes, total_bytes);
+}
+
 // Footprints (ow, dw, fw per axis from the n values, all n^6 of them) on
 // which the main pass's size test (foot_width) and the second pass's
 // (min_width, as the reference has it) decide differently for some of the
