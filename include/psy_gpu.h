@@ -249,6 +249,11 @@ int psy_ctx_destroy(psy_ctx* ctx);
 #define PSY_TRACE_MODE_COHERENT 2
 #define PSY_TRACE_MODE_PLAIN_COHERENT 3
 int psy_ctx_set_trace_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_per_cu);
+/* Gives the choice of the main pass's form and of its continuations (below)
+ * back to the library after psy_ctx_set_trace_mode, psy_ctx_set_continuation
+ * or psy_render_autotune: as on a new context (no counterpart in the
+ * reference). */
+int psy_ctx_reset_trace_form(psy_ctx* ctx);
 /* Main-pass traversal stack in LDS (no counterpart in the reference, whose
  * BitStack and node stack live in CPU memory): 16 entries (default, 5 waves
  * per SIMD) or 32 (2 waves per SIMD).  A ray whose stack outgrows them keeps
@@ -530,8 +535,9 @@ int psy_film_adaptive(psy_ctx* ctx, const float* sample_xyz, int32_t width, int3
  * chunks, up to the full spp), the whole image as 2 to 4 chunks all in
  * flight and the shading kernel's register budget
  * (psy_ctx_set_render_shade_waves), and leaves the fastest setting on the
- * context
- * and the scene.  `out` (or NULL) receives it. */
+ * context and the scene; where that is the main pass's own choice of form,
+ * the context keeps the choice and trace_mode says what it is for this
+ * scene.  `out` (or NULL) receives it. */
 typedef struct psy_render_tuning {
     int32_t mode;             /* PSY_RENDER_STREAM or PSY_RENDER_WAVEFRONT */
     int32_t trace_mode;       /* PSY_TRACE_MODE_*                        */

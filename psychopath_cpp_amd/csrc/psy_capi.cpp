@@ -270,6 +270,15 @@ int psy_ctx_set_trace_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_pe
     return PSY_OK;
 }
 
+int psy_ctx_reset_trace_form(psy_ctx* ctx) {
+    if (!ctx) return fail(PSY_ERR_INVALID, "psy_ctx_reset_trace_form: NULL context");
+    ctx->mode = psy_ctx::MODE_DEFAULT;
+    ctx->refill_min = psy_ctx::DEFAULT_REFILL_MIN;
+    ctx->blocks_per_cu = 0;
+    ctx->cont_below = psy_ctx::CONT_DEFAULT;
+    return PSY_OK;
+}
+
 int psy_ctx_set_render_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_per_cu) {
     if (!ctx) return fail(PSY_ERR_INVALID, "psy_ctx_set_render_mode: NULL context");
     if (mode != PSY_RENDER_WAVEFRONT && mode != PSY_RENDER_FUSED && mode != PSY_RENDER_STREAM)

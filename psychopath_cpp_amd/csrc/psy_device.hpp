@@ -137,6 +137,18 @@ struct DevLights {
     int32_t n_asms;
 };
 
+// The form the main pass takes by default, one thread per ray: coherent for
+// world rays in a moving scene of patches.  A BVH step there reads the nodes'
+// changes and starts walks in instances' own spaces, so that a round that
+// issues it beside a walk for 14 lanes each is dear: 960x540 moving bicubic
+// spheres 0.59 ms for 0.70, their render at 8 samples 14.7 for 17.2, smaller
+// grids and images 6 to 16 % less; static patches with one moving sphere
+// (64x64 heightfield) 427 us for 467, the render at 512x512x4 5.29 ms for
+// 5.59.  Elsewhere a round of one kind costs as much as it saves or more:
+// static patches 9 % less to 3 % more, spheres and lights 1 to 17 % more,
+// object rays 5 % more.
+inline bool coherent_pays(const DevScene& s, bool world) { return world && s.bvh1 && s.mostly_patches != 0; }
+
 // ---- launchers (psy_kernels.hip) -------------------------------------------
 int launch_build_dice(const float* odata, const DevObject* objs, const int32_t* patch_ids,
                       int n_patches, int levels, float4* dice, hipStream_t st);
@@ -158,7 +170,7 @@ struct TraceTuning {
     bool persistent;
     bool coherent = false;  // persistent: step one kind of work per wave step
     bool plain_coherent = false;  // one thread per ray, stepping one kind of work per wave step
-    bool auto_form = false;       // one thread per ray, stepped so where that pays (launch_trace_w)
+    bool auto_form = false;       // one thread per ray, stepped so where that pays (coherent_pays)
     int persist_blocks;    // persistent grid with the 16-entry stack
     int persist_blocks32;  // and with the 32-entry stack
     int refill_min;

@@ -117,10 +117,10 @@ struct psy_ctx {
     static constexpr int CONT_DEFAULT = -1, DEFAULT_CONT_BELOW = 24;
     int cont_below = CONT_DEFAULT;
     // main-pass form: MODE_DEFAULT (plain, or plain coherent where that pays:
-    // launch_trace_w) until psy_ctx_set_trace_mode picks one
-    static constexpr int MODE_DEFAULT = -1;
+    // coherent_pays) until psy_ctx_set_trace_mode picks one
+    static constexpr int MODE_DEFAULT = -1, DEFAULT_REFILL_MIN = 16;
     int mode = MODE_DEFAULT;
-    int refill_min = 16;
+    int refill_min = DEFAULT_REFILL_MIN;
     int blocks_per_cu = 0;  // <= 0: from occupancy
     // pass timing: event triples of the trace calls since the last query
     bool timing = false;

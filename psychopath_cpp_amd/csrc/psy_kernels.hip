@@ -836,15 +836,7 @@ static int launch_trace_w(const DevScene& s, int stack_need, const float* rays, 
     const int64_t plain_blocks = grid_for(n, TRACE_BLOCK);
     const int64_t persist_blocks = (int64_t)(tune.stack > 16 ? tune.persist_blocks32 : tune.persist_blocks);
     const int refill = std::max(1, std::min(64, tune.refill_min));
-    // World rays in a moving scene of patches: one kind of step a round.  A
-    // BVH step there reads the nodes' changes and starts walks in instances'
-    // own spaces, so that a round that issues it beside a walk for 14 lanes
-    // each is dear: 960x540 moving bicubic spheres 0.59 ms for 0.70, their
-    // render at 8 samples 14.7 for 17.2, smaller grids and images 6 to 16 %
-    // less.  Elsewhere a round of one kind costs as much as it saves or more:
-    // static patches 9 % less to 3 % more, spheres and lights 1 to 17 % more,
-    // object rays 5 % more.
-    const bool coherent = tune.plain_coherent || (W && tune.auto_form && s.bvh1 && s.mostly_patches != 0);
+    const bool coherent = tune.plain_coherent || (tune.auto_form && coherent_pays(s, W));
     if (tune.persistent && persist_blocks > 0 && persist_blocks < plain_blocks) {
         if (tune.stack > 16)
             hipLaunchKernelGGL((k_trace_persist<W, 32>), dim3((unsigned)persist_blocks), dim3(TRACE_BLOCK), 0, st, s,

@@ -886,7 +886,8 @@ int psy_render_adaptive(psy_ctx* ctx, const psy_scene* s, const psy_render_param
 // paths in flight (wavefront chunk or stream pool), the main pass's launch
 // form and LDS stack depth, and the stream form's steps per captured graph,
 // timing psy_render on a sample budget of the image (every pixel at reduced
-// spp).  Leaves the best setting on the context.
+// spp).  Leaves the best setting on the context; where that is the main
+// pass's own choice of form, the choice, which other scenes then have too.
 int psy_render_autotune(psy_ctx* ctx, psy_scene* s, const psy_render_params* prm, int64_t max_samples,
                         psy_render_tuning* out) {
     if (int rc = check_render(ctx, s, prm, "psy_render_autotune")) return rc;
@@ -940,7 +941,8 @@ int psy_render_autotune(psy_ctx* ctx, psy_scene* s, const psy_render_params* prm
         ++trials;
         return PSY_OK;
     };
-    Cfg best{PSY_RENDER_STREAM, std::min<int64_t>((int64_t)1 << 21, total), PSY_TRACE_MODE_PLAIN, 16, 16, 4, 2, 0};
+    Cfg best{PSY_RENDER_STREAM, std::min<int64_t>((int64_t)1 << 21, total), psy_ctx::MODE_DEFAULT,
+             psy_ctx::DEFAULT_REFILL_MIN, 16, 4, 2, 0};
     double best_m = 0.0;
     int rc = timed(best, &best_m);
     auto consider = [&](Cfg c) -> int {
@@ -962,7 +964,12 @@ int psy_render_autotune(psy_ctx* ctx, psy_scene* s, const psy_render_params* prm
     }
     if (!rc) { Cfg t = best; t.tmode = PSY_TRACE_MODE_PERSISTENT; t.refill = 32; rc = consider(t); }
     if (!rc) { Cfg t = best; t.stack = 32; rc = consider(t); }
-    if (!rc && best.tmode == PSY_TRACE_MODE_PLAIN) { Cfg t = best; t.tmode = PSY_TRACE_MODE_PLAIN_COHERENT; rc = consider(t); }
+    // the one-thread-per-ray form that the library would not take by itself
+    const int own_form = ctx->cont_below == psy_ctx::CONT_DEFAULT && coherent_pays(s->dev, true)
+                             ? PSY_TRACE_MODE_PLAIN_COHERENT
+                             : PSY_TRACE_MODE_PLAIN;
+    const int other_form = own_form == PSY_TRACE_MODE_PLAIN ? PSY_TRACE_MODE_PLAIN_COHERENT : PSY_TRACE_MODE_PLAIN;
+    if (!rc && best.tmode == psy_ctx::MODE_DEFAULT) { Cfg t = best; t.tmode = other_form; rc = consider(t); }
     if (best.mode == PSY_RENDER_STREAM)
         for (int it : {2, 8, 16}) if (!rc && it != best.iters) { Cfg t = best; t.iters = it; rc = consider(t); }
     // wavefront chunks in flight: 1, 3 and 4 against the search's 2, then
@@ -987,9 +994,9 @@ int psy_render_autotune(psy_ctx* ctx, psy_scene* s, const psy_render_params* prm
         // chunks in flight favour the 16-entry stack's higher occupancy)
         if (!rc) { Cfg t = best; t.stack = best.stack == 16 ? 32 : 16; rc = consider(t); }
         // and the other one-thread-per-ray launch form
-        if (!rc && (best.tmode == PSY_TRACE_MODE_PLAIN || best.tmode == PSY_TRACE_MODE_PLAIN_COHERENT)) {
+        if (!rc && best.tmode != PSY_TRACE_MODE_PERSISTENT) {
             Cfg t = best;
-            t.tmode = best.tmode == PSY_TRACE_MODE_PLAIN ? PSY_TRACE_MODE_PLAIN_COHERENT : PSY_TRACE_MODE_PLAIN;
+            t.tmode = best.tmode == psy_ctx::MODE_DEFAULT ? other_form : psy_ctx::MODE_DEFAULT;
             rc = consider(t);
         }
     }
@@ -1023,7 +1030,7 @@ int psy_render_autotune(psy_ctx* ctx, psy_scene* s, const psy_render_params* prm
     apply(best);
     if (out) {
         out->mode = best.mode;
-        out->trace_mode = best.tmode;
+        out->trace_mode = best.tmode == psy_ctx::MODE_DEFAULT ? own_form : best.tmode;
         out->refill_min = best.refill;
         out->stack = best.stack;
         out->steps_per_graph = best.iters;

@@ -36,6 +36,7 @@ def lib():
     L.psy_ctx_create.argtypes = [C.c_int, C.POINTER(vp)]
     L.psy_ctx_destroy.argtypes = [vp]
     L.psy_ctx_set_trace_mode.argtypes = [vp, C.c_int, C.c_int, C.c_int]
+    L.psy_ctx_reset_trace_form.argtypes = [vp]
     L.psy_ctx_retrace_count.argtypes = [vp, C.POINTER(i64)]
     L.psy_ctx_trace_pass_counts.argtypes = [vp, C.POINTER(i64), C.POINTER(i64)]
     L.psy_ctx_set_render_chunk.argtypes = [vp, i64]
@@ -146,6 +147,10 @@ class Context:
         if persistent:
             mode = abi.PSY_TRACE_MODE_COHERENT if coherent else abi.PSY_TRACE_MODE_PERSISTENT
         check(lib().psy_ctx_set_trace_mode(self.handle, mode, refill_min, blocks_per_cu), "psy_ctx_set_trace_mode")
+
+    def reset_trace_form(self):
+        """psy_ctx_reset_trace_form: the main pass's form and continuations as on a new context."""
+        check(lib().psy_ctx_reset_trace_form(self.handle), "psy_ctx_reset_trace_form")
 
     def set_trace_stack(self, entries):
         """psy_ctx_set_trace_stack: main-pass LDS stack entries (16 or 32)."""

@@ -51,6 +51,8 @@ def lib():
     L.hb_scene_stack_need.argtypes = [C.POINTER(abi.SceneDesc), C.c_int, C.POINTER(C.c_int)]
     L.hb_foot_mismatches.argtypes = [vp, C.c_int, vp, C.c_int, vp, C.c_int, C.c_float, C.c_float, vp]
     L.hb_foot_mismatches.restype = i64
+    L.hb_trace_form.argtypes = [C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int)]
+    L.hb_trace_form.restype = None
     L.hb_take_slots.argtypes = [C.c_int, C.c_int, C.POINTER(C.c_int), C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int),
                                 C.POINTER(C.c_int)]
     L.hb_slots_that_fit.argtypes = [C.c_int, C.POINTER(i64), i64, i64]
@@ -80,6 +82,14 @@ def trace(scene_py, rays, world=True, dice_depth=10, occlusion_only=False, threa
     if rc != 0:
         raise RuntimeError(f"hb_trace failed with status {rc}")
     return {"t": t, "inst": inst, "u": u, "v": v, "aux": aux, "retraced": rt.value}
+
+
+def trace_form(steps):
+    """A context's main-pass form after `steps` ("mode", "continuation", "reset"): see hb_trace_form."""
+    ids = [("mode", "continuation", "reset").index(x) for x in steps]
+    out = (C.c_int * 6)()
+    lib().hb_trace_form((C.c_int * max(1, len(ids)))(*ids), len(ids), out)
+    return tuple(out)
 
 
 def take_slots(want, need, held, room, error=0):

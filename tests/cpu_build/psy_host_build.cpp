@@ -132,6 +132,20 @@ int hb_scene_stack_need(const psy_scene_desc* d, int dice_depth, int* need) {
 // Waves of the second pass's wave-per-ray kernel in a call of n rays.
 int64_t hb_second_pass_waves(int64_t n) { return (int64_t)coop_blocks(n) * (TRACE_BLOCK / 64); }
 
+// The main pass's form on a context, as (mode, refill, blocks, continue
+// below, own choice for object rays, for world rays): after each of `steps`
+// (0 set the mode, 1 set the continuation, 2 reset).  No device call is made.
+void hb_trace_form(const int* steps, int n_steps, int* out) {
+    psy_ctx c;
+    for (int k = 0; k < n_steps; ++k) {
+        if (steps[k] == 0) psy_ctx_set_trace_mode(&c, PSY_TRACE_MODE_PERSISTENT, 32, 3);
+        if (steps[k] == 1) psy_ctx_set_continuation(&c, 8);
+        if (steps[k] == 2) psy_ctx_reset_trace_form(&c);
+    }
+    const int v[6] = {c.mode, c.refill_min, c.blocks_per_cu, c.cont_below, c.tuning(false).auto_form, c.tuning(true).auto_form};
+    for (int k = 0; k < 6; ++k) out[k] = v[k];
+}
+
 // A render's memory, in units: room for `room`, of which chunks beyond the
 // first hold held[k] from an earlier render and every chunk of this one needs
 // `need`.  Returns the hipError_t, the chunks it got and how often it asked.
