@@ -462,9 +462,9 @@ def test_gpu_c1_full_stream(c1, oracle):
 def test_gpu_long_second_pass_queue(oracle):
     """Camera rays at 1024 x 1024 over the sphere scene: the ground patch
     dices below its 24 cached levels for a large share of them, so the
-    second pass walks a queue of thousands of rays (its wide build, 2 waves
-    per SIMD, takes queues of 4096 or more); a random sample of 4096 rays
-    matches the oracle."""
+    second pass works a queue of thousands of rays (a lane per ray, as it does
+    queues of 1024 or more); a random sample of 4096 rays matches the
+    oracle."""
     sc = configs.sphere_scene()
     o = oracle.OracleScene(sc)
     ctx = gpu.Context(0)
@@ -493,8 +493,8 @@ def test_gpu_long_second_pass_queue(oracle):
         say("long queue sample: ids agree", same_id.mean(), "t within 1e-5", t_ok.mean())
         assert hit_o.mean() > 0.3
         assert same_id.mean() >= 0.9999 and t_ok.mean() >= 0.9999
-        # the same queue through the narrow build alone and the wide build
-        # alone: the same hits bit for bit; with a node budget of 1 and 4
+        # the same queue a wave per ray and a lane per ray: the same hits bit
+        # for bit; with a node budget of 1 and 4
         # expansions most second-pass rays finish in the third,
         # wave-cooperative pass, whose lanes merge hits in another order
         # (exact ties may resolve differently): the same closest hits

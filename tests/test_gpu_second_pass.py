@@ -31,9 +31,14 @@ def test_gpu_second_pass_forms_agree(name, depth):
                 second, third = ctx.pass_counts()
                 assert second == queued
                 assert third == 0 or wide_min <= queued
+                # a lane's ray that needs more than one node expansion is handed over
+                assert third > 0 or wide_min > queued or budget > 1
                 # exactly tied micropolygons may resolve differently; distances do not depend on the form
                 assert torch.equal(h.t, ref.t)
-                assert float((h.inst == ref.inst).float().mean()) >= 0.9999
+                same = h.inst == ref.inst
+                for k in ("u", "v", "aux"):
+                    same &= getattr(h, k) == getattr(ref, k)
+                assert float(same.float().mean()) >= 0.9999
                 occ = gpu.trace_world(ctx, g, w, occlusion_only=True)
                 assert torch.equal(occ.inst != -1, ref.inst != -1)
         g.close()
