@@ -256,8 +256,10 @@ int psy_ctx_set_trace_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_pe
 int psy_ctx_reset_trace_form(psy_ctx* ctx);
 /* Main-pass traversal stack in LDS (no counterpart in the reference, whose
  * BitStack and node stack live in CPU memory): 16 entries (default, 5 waves
- * per SIMD) or 32 (2 waves per SIMD).  A ray whose stack outgrows them keeps
- * the rest in the context's scratch.  Results are identical. */
+ * per SIMD) or 32 (2 waves per SIMD).  In a scene with patches a ray whose
+ * stack outgrows them keeps the rest in the context's scratch while that has
+ * room; any other such ray is retraced by the second pass.  Results are
+ * identical. */
 int psy_ctx_set_trace_stack(psy_ctx* ctx, int entries);
 /* The trace's second pass (no counterpart in the reference, which splits
  * patches per ray batch without a cache): rays that the main pass hands on
@@ -265,7 +267,10 @@ int psy_ctx_set_trace_stack(psy_ctx* ctx, int entries);
  * wide_min rays or more (default 1024; 0: always a lane each; UINT32_MAX:
  * always a wave each); a lane's ray that takes more than `budget` (>= 1,
  * default 512) split-tree node expansions, or many cache nodes, goes on to
- * the third pass, a wave each.  Results do not depend on either setting. */
+ * the third pass, a wave each.  Hits do not depend on either setting, but
+ * for micropolygons at exactly the same distance, of which a lane and a wave
+ * may report different ones; the form goes by the queue's length, so how
+ * rays are split into calls or chunks can decide such a tie too. */
 int psy_ctx_set_second_pass(psy_ctx* ctx, uint32_t wide_min, int32_t budget);
 /* The main pass's continuations (no counterpart in the reference, whose
  * lanes are CPU threads): the rays of one 64-lane wave end after very
@@ -325,13 +330,15 @@ int psy_ctx_set_render_mode(psy_ctx* ctx, int mode, int refill_min, int blocks_p
 /* Steps per captured graph of PSY_RENDER_STREAM: even, 2..64 (default 4). */
 int psy_ctx_set_stream_steps(psy_ctx* ctx, int steps_per_graph);
 /* Rays of the latest trace call on this context that the main pass handed
- * to the second pass (split below the dice cache, or a direction the main
- * pass does not take).  Synchronizes the device; for diagnostics. */
+ * to the second pass: they split below the dice cache, their stack outgrew
+ * the main pass's (psy_ctx_set_trace_stack), or their direction has no
+ * finite inverse, in the world's space or in a patch's.  Synchronizes the
+ * device; for diagnostics. */
 int psy_ctx_retrace_count(psy_ctx* ctx, int64_t* out);
 /* Rays of the latest trace call (psy_trace_*, or the last step of a
- * psy_render on the caller's stream) that took the second pass, and those of them that ran out of
- * its split budget and took the third, wave-cooperative pass.  Synchronizes
- * the device. */
+ * psy_render on the caller's stream) that took the second pass, and those of
+ * them that outran its limits and took the third, wave-cooperative pass
+ * (psy_ctx_set_second_pass).  Synchronizes the device. */
 int psy_ctx_trace_pass_counts(psy_ctx* ctx, int64_t* second, int64_t* third);
 /* Pass timing (no counterpart in the reference): while enabled, each trace
  * call records HIP events on its stream around the main pass and the

@@ -121,6 +121,12 @@ __global__ __launch_bounds__(TRACE_BLOCK, main_waves(WORLD, STACK)) void k_trace
     if (lane_finish(s, L, h)) enqueue_second(queue, heads, counters, L);
 }
 
+// Main pass, persistent: a grid that fills the GPU once; every wave claims
+// rays from a global counter (counters[2..3], u64) 256 at a time (one atomic
+// per claim) and refills its finished lanes from its claim whenever at least
+// `refill_min` of them are idle, so the wave's lanes stay busy through the
+// long tail of incoherent rays.  Every wave leaves once the counter has
+// passed n and its lanes are idle.
 constexpr int PERSIST_CHUNK = 256;
 
 template <bool WORLD, int STACK>

@@ -967,8 +967,9 @@ PSY_DEV bool trace_one(const DevScene& s, const float* __restrict__ rays, int64_
 // independently instead of waiting at every BVH leaf for the longest
 // split-tree walk in the wave.  Rays that reach the bottom of the dice cache
 // with a node still to split are handed to the second pass.  A BVH stack
-// that outgrows the main pass's MAIN_STACK entries of LDS keeps its bottom
-// in the trace's scratch pool (stack_spill).
+// that outgrows the main pass's entries of LDS keeps its bottom in the
+// trace's scratch pool (stack_spill) in a scene with patches; without, and
+// with the pool used up, its ray is handed on too.
 // ---------------------------------------------------------------------------
 #ifndef PSY_MAIN_STACK
 #define PSY_MAIN_STACK 16
@@ -978,8 +979,8 @@ PSY_DEV bool trace_one(const DevScene& s, const float* __restrict__ rays, int64_
 #endif
 constexpr int MAIN_STACK = PSY_MAIN_STACK;
 // The main pass also comes with a 32-entry stack at lower occupancy (fewer
-// rays handed to the second pass on deep hierarchies); waves per SIMD of
-// each form, as launch bounds.
+// stacks outgrow it on deep hierarchies); waves per SIMD of each form, as
+// launch bounds.
 constexpr int main_waves(bool world, int stack, bool coherent = false) {
     return stack <= 16 ? ((world || coherent) ? 4 : PSY_MAIN_WAVES_PER_SIMD) : 2;
 }
@@ -1078,7 +1079,13 @@ PSY_DEV uint32_t wave_alloc(uint32_t* counter, uint32_t want) {
 // second pass meant retracing each from the root, one to a wave, at the end
 // of the call: about 1 ms of latency per step.  That render went from 33.2
 // to 19.0 ms (with world rays no longer continued), one frame of its camera
-// rays at 960x540 from 1.27 to 0.76 ms.
+// rays at 960x540 from 1.27 to 0.76 ms.  A chunk is not used twice, so that a
+// stack that shrinks and grows about the LDS limit soon uses the pool up
+// where many do: then the rest is retraced, and that is the better way for
+// many.  With a place of its own for each ray, 1024 nested spheres over a
+// patch took 1.95 ms for 128x128 rays (3.99 as it is), but 24.2 for
+// 1450x1450 (14.1): rays that outlive their wave run alone in it, while the
+// second pass packs them.
 PSY_DEV bool stack_spill(Lane& L, int32_t (*stk_ref)[TRACE_BLOCK], float (*stk_near)[TRACE_BLOCK], int tid,
                          const DeepPool& P) {
     if (P.cap < SPILL_POOL) return false;
@@ -1380,7 +1387,8 @@ PSY_DEV bool lane_step(const DevScene& s, Lane& L, int32_t (*stk_ref)[TRACE_BLOC
         cmpswap(k1, r1, k2, r2);
         const int npush = (k1 < INFINITY ? 1 : 0) + (k2 < INFINITY ? 1 : 0) + (k3 < INFINITY ? 1 : 0);
         // a scene without patches hands such a ray to the second pass, where
-        // a few nodes and shapes are soon retraced
+        // nodes and shapes are soon retraced (1024 nested spheres: 32x32 rays
+        // 2.54 ms, with the pool 2.67, 512x512 4.48 and 4.55)
         if (L.sp + npush > STACK && !(s.dice && stack_spill(L, stk_ref, stk_near, tid, P))) {
             L.state |= LANE_RETRACE;
             return true;
@@ -1695,20 +1703,6 @@ __device__ void resume_list_coop(const DevScene& s, const float* __restrict__ ra
     }
     if (b.inst != before || b.t != t_before) resume_store(h, i, b);
 }
-
-// Main pass, one thread per ray.
-
-// Main pass, persistent: a grid that fills the GPU once; every wave claims
-// rays from a global counter 256 at a time (one atomic per claim) and
-// refills its finished lanes from its claim whenever at least `refill_min`
-// of them are idle, so the wave's lanes stay busy through the long tail of
-// incoherent rays.  Every wave leaves once the counter has passed n and its
-// lanes are idle.
-
-// Second pass: retrace the queued rays with subdivision below the cache and
-// a stack of STACK >= the scene's worst case.
-
-// counters[0]: retrace queue length; counters[2..3]: next ray (u64)
 
 // ---------------------------------------------------------------------------
 // WorldRay::to_ray over a stream (basics/ray.hpp:207-252, :310-323)
