@@ -115,8 +115,8 @@ struct psy_ctx {
     // all in world form, 1 to 20 % less: spheres 256x256x16 1.62 ms for 2.01,
     // heightfield 1024x1024x16 51.9 for 52.9).  World streams of 2^20 to
     // 2^22 rays over static patches take it both ways: camera rays 2 to 23 %
-    // less without, camera and bounce rays mixed over finely diced ground 14
-    // to 18 % less, but bounce rays alone 0 to 6 % more, and 2 to 7 % more
+    // less without, camera and bounce rays mixed over finely diced ground 13
+    // to 18 % less, but bounce rays alone 0 to 7 % more, and 2 to 8 % more
     // with the occlusion flag (2^22 over subdivision surfaces 2.67 ms for
     // 2.51): a program that traces many such sets the limit by hand.
     // Letting the waves of spread-out rays alone continue gave those back,
