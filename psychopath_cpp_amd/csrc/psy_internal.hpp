@@ -24,9 +24,11 @@ int floats_per_kind(int kind);
             return ::psy::fail(PSY_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// The status, with its message, of an allocation that returned `e`.
+// The status, with its message, of an allocation (and the synchronization
+// before it) that returned `e`.
 inline int alloc_status(hipError_t e) {
-    return e == hipSuccess ? PSY_OK : fail(PSY_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
+    return e == hipSuccess ? PSY_OK
+                           : fail(PSY_ERR_HIP, std::string("allocating device memory: ") + hipGetErrorString(e));
 }
 
 // Owning device allocation.

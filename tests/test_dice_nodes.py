@@ -79,6 +79,32 @@ def test_footprints_that_are_not_finite_stay_in_the_main_pass(planes, value):
         assert np.array_equal(a[k], b[k]), k
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("planes", [(8, 9), (10, 11), (8, 9, 10, 11, 12, 13), (8,), (11,)])
+def test_gpu_infinite_footprints_stay_in_the_main_pass(planes):
+    import torch
+    from psychopath_cpp_amd import gpu
+    rays = _object_rays(600, 0.05)
+    rays[10:12] = 0.01
+    for p in planes:
+        rays[p] = np.inf
+    rays[2, ::2] = 0.05
+    x = torch.from_numpy(rays).cuda()
+    ctx = gpu.Context(0)
+    try:
+        got = []
+        for depth in (14, 0):
+            g = gpu.GpuScene(ctx, _scene("bilinear", min_upoly=0.02), dice_depth=depth)
+            h = gpu.trace_rays(ctx, g, x)
+            got.append([y.clone() for y in (h.t, h.inst, h.u, h.v, h.aux)])
+            assert depth == 0 or ctx.retrace_count() == 0
+            g.close()
+        assert int((got[0][1] == 0).sum()) > 100
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("rate", [0.25, 1.0])
 @pytest.mark.parametrize("min_upoly", [0.0, 1e-5, 0.5])
 def test_size_test_is_the_references_for_every_footprint(rate, min_upoly):
